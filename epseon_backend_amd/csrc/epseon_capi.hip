@@ -1338,6 +1338,20 @@ const BandWindow* scan_window_set(const epseon_ctx* ctx)
     return ctx->scan_windows ? ctx->d_win_band : ctx->d_win_full;
 }
 
+// Wavefronts per scan workgroup.  Whole-grid scans with at most a few
+// wavefronts per SIMD take their time from the fullest SIMD, and one-wavefront
+// workgroups pile up on some SIMDs depending on what ran before; workgroups of
+// four put one wavefront on each SIMD of a compute unit.  Measured on 8 x
+// 200,000 points x 16,384 energies (two wavefronts per SIMD) after a load:
+// 4.9 -> 3.3 ms per scan; with one per SIMD or less within 2 %.  Longer scans
+// (and windowed ones, whose wavefronts differ) keep the tuning's value: the
+// SIMDs take new wavefronts as others end.
+int32_t scan_waves_per_block(const epseon_ctx* ctx)
+{
+    const bool few = static_cast<int64_t>(ctx->n_scan_tasks) < kWindowsMinScanWavesPerSimd * 4 * ctx->compute_units;
+    return ctx->waves_per_block == 1 && !ctx->scan_windows && few ? 4 : ctx->waves_per_block;
+}
+
 // Scan of the potentials [k0, k1) in task order on `stream`; the whole batch
 // goes through the per-XCD bins.
 hipError_t run_scan(epseon_ctx* ctx, hipStream_t stream, size_t k0, size_t k1)
@@ -1345,17 +1359,18 @@ hipError_t run_scan(epseon_ctx* ctx, hipStream_t stream, size_t k0, size_t k1)
     const int32_t t0 = ctx->cum_scan_tasks[k0];
     const int32_t t1 = ctx->cum_scan_tasks[k1];
     const BandWindow* win = scan_window_set(ctx);
+    const int32_t waves = scan_waves_per_block(ctx);
     if (ctx->xcd_scan && k0 == 0 && k1 == ctx->cum_scan_tasks.size() - 1) {
         if (ctx->scan_windows)
             return launch_scan(stream, ctx->d_ut, ctx->d_rec, win, ctx->d_xcd_scan_tasks_band, t1 - t0,
-                               ctx->d_xcd_bins_band, ctx->xcd_max_bin_band, ctx->waves_per_block,
+                               ctx->d_xcd_bins_band, ctx->xcd_max_bin_band, waves,
                                ctx->d_nodes, ctx->d_far, ctx->d_resc);
         return launch_scan(stream, ctx->d_ut, ctx->d_rec, win, ctx->d_xcd_scan_tasks, t1 - t0,
-                           ctx->d_xcd_bins, ctx->xcd_max_bin, ctx->waves_per_block, ctx->d_nodes,
+                           ctx->d_xcd_bins, ctx->xcd_max_bin, waves, ctx->d_nodes,
                            ctx->d_far, ctx->d_resc);
     }
     return launch_scan(stream, ctx->d_ut, ctx->d_rec, win, ctx->d_scan_tasks + t0, t1 - t0, nullptr, 0,
-                       ctx->waves_per_block, ctx->d_nodes, ctx->d_far, ctx->d_resc);
+                       waves, ctx->d_nodes, ctx->d_far, ctx->d_resc);
 }
 
 // Make `stream` wait for the segment tables of the last load (once), and,
