@@ -27,9 +27,9 @@ namespace epseon::hip {
 static_assert(kBands == EPSEON_BANDS, "band count of the C ABI");
 
 hipError_t launch_shift_potential(hipStream_t, const double*, const PotentialRecord*, int32_t,
-                                  int32_t, double*, double*, double*);
-hipError_t launch_potential_stats(hipStream_t, const double*, const int64_t*, const int64_t*,
-                                  const double*, int32_t, PotentialStats*);
+                                  int32_t, double*, double*, double*, ChunkEdge*);
+hipError_t launch_potential_stats(hipStream_t, const double*, const int64_t*, const int64_t*, const int32_t*,
+                                  const double*, int32_t, int32_t, ChunkMin*, PotentialStats*);
 hipError_t launch_scan(hipStream_t, const double*, const PotentialRecord*, const BandWindow*,
                        const WaveTask*, int32_t, const int32_t*, int32_t, int32_t, int32_t*, double*,
                        int32_t*);
@@ -44,7 +44,8 @@ hipError_t launch_refine_segmented(hipStream_t, int32_t, int32_t, const double*,
                                    double*, int32_t*, int32_t*, int32_t*);
 hipError_t launch_segment_tables(hipStream_t, const double*, const PotentialRecord*, const TableJob*,
                                  int32_t, int32_t, double*);
-hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord*, int32_t, int2*);
+hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord*, int32_t, int64_t,
+                               const ChunkEdge*, int2*);
 hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, int32_t, const int32_t*, const int32_t*,
                                 const int32_t*, int64_t*);
 hipError_t launch_normalize(hipStream_t, const double*, const double*, const PotentialRecord*,
@@ -277,7 +278,6 @@ struct epseon_ctx {
     std::vector<epseon_potential_desc> desc;
     std::vector<PotentialRecord> rec;
     int64_t total_points = 0, total_energies = 0, total_levels = 0;
-    int32_t max_points = 0;
 
     double* d_v = nullptr;
     double* d_ut = nullptr;
@@ -723,7 +723,11 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     char msg[256];
     // Descriptor checks (no V access).
     std::vector<double> betas(static_cast<size_t>(std::max(count, 1)));
-    int64_t user_span = 0;
+    // Chunks of the statistics and table passes before each potential.
+    std::vector<int32_t> stats_chunk0(static_cast<size_t>(std::max(count, 1)));
+    std::vector<int32_t> table_chunk0(static_cast<size_t>(std::max(count, 1)));
+    int64_t user_span = 0, all_points = 0;
+    int32_t stats_chunks = 0, table_chunks = 0, max_stats_chunks = 0, max_table_chunks = 0;
     for (int32_t p = 0; p < count; ++p) {
         const epseon_potential_desc& d = desc[p];
         if (d.n_points < 4 || d.n_points > (int64_t(1) << 30)) {
@@ -755,6 +759,14 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         const double h = (d.r_max - d.r_min) / static_cast<double>(d.n_points - 1);
         betas[static_cast<size_t>(p)] = (h * h * d.reduced_mass) / (12.0 * kHbar2Over2Amu);
         user_span = std::max<int64_t>(user_span, v_offsets[p] + d.n_points);
+        all_points += d.n_points;
+        const int32_t sc = load_chunks(d.n_points, kStatsChunk), tc = load_chunks(d.n_points, kTableChunk);
+        stats_chunk0[static_cast<size_t>(p)] = stats_chunks;
+        table_chunk0[static_cast<size_t>(p)] = table_chunks;
+        stats_chunks += sc;
+        table_chunks += tc;
+        max_stats_chunks = std::max(max_stats_chunks, sc);
+        max_table_chunks = std::max(max_table_chunks, tc);
     }
 
     // V statistics: min V, its first index, the wall-trimmed Dirichlet points
@@ -799,24 +811,31 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         int64_t* d_cnt = nullptr;
         double* d_beta = nullptr;
         PotentialStats* d_st = nullptr;
+        int32_t* d_chunk0 = nullptr;
+        ChunkMin* d_chunks = nullptr;
         EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_off));
         EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_cnt));
         EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_beta));
         EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_st));
+        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_chunk0));
+        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(stats_chunks), &d_chunks));
         EPSEON_HIP_TRY(hipMemcpyAsync(d_off, v_offsets, count * sizeof(int64_t), hipMemcpyHostToDevice,
                                       ctx->stream));
         EPSEON_HIP_TRY(hipMemcpyAsync(d_cnt, counts.data(), count * sizeof(int64_t),
                                       hipMemcpyHostToDevice, ctx->stream));
         EPSEON_HIP_TRY(hipMemcpyAsync(d_beta, betas.data(), count * sizeof(double),
                                       hipMemcpyHostToDevice, ctx->stream));
-        EPSEON_HIP_TRY(launch_potential_stats(ctx->stream, v_dev, d_off, d_cnt, d_beta, count, d_st));
+        EPSEON_HIP_TRY(hipMemcpyAsync(d_chunk0, stats_chunk0.data(), count * sizeof(int32_t), hipMemcpyHostToDevice,
+                                      ctx->stream));
+        EPSEON_HIP_TRY(launch_potential_stats(ctx->stream, v_dev, d_off, d_cnt, d_chunk0, d_beta, count,
+                                              max_stats_chunks, d_chunks, d_st));
         EPSEON_HIP_TRY(hipMemcpyAsync(vstats.data(), d_st, count * sizeof(PotentialStats),
                                       hipMemcpyDeviceToHost, ctx->stream));
         EPSEON_HIP_TRY(hipStreamSynchronize(ctx->stream));
     }
 
     int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0;
-    int32_t max_points = 0, max_seg_rows = 0;
+    int32_t max_seg_rows = 0;
     double scan_pu = 0.0;
     for (int32_t p = 0; p < count; ++p) {
         const epseon_potential_desc& d = desc[p];
@@ -879,6 +898,7 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         r.psi_segs_left = (r.match + r.psi_seg_len - 1) / r.psi_seg_len;
         r.psi_segs_right = (r.n_points - 2 - r.match + r.psi_seg_len - 1) / r.psi_seg_len;
         r.psi_ckpt = ckpt_total;
+        r.chunk0 = table_chunk0[static_cast<size_t>(p)];
         if (r.flags == EPSEON_POT_OK)
             ckpt_total += static_cast<int64_t>(d.level_count) * (r.psi_segs_left + r.psi_segs_right);
         r.user_offset = v_offsets[p];
@@ -893,14 +913,12 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         pts += ((d.n_points + 7) & ~int64_t(7)) + 64;
         en += d.n_energies;
         lv += d.level_count;
-        max_points = std::max(max_points, static_cast<int32_t>(d.n_points));
         if (r.flags == EPSEON_POT_OK)
             scan_pu += static_cast<double>(r.n_points - 2) * static_cast<double>(d.n_energies);
     }
     ctx->total_points = pts;
     ctx->total_energies = en;
     ctx->total_levels = lv;
-    ctx->max_points = max_points;
     ctx->scan_pu_full = scan_pu;
     ctx->user_span = user_span;
     ctx->psi_total = psi_total;
@@ -1023,6 +1041,8 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     const size_t nw = std::max<size_t>(static_cast<size_t>(count) * kBands, 1);
     int2* d_raw_windows = nullptr;
     EPSEON_HIP_TRY(arena_array(a, nw, &d_raw_windows));
+    ChunkEdge* d_edges = nullptr;
+    EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max(table_chunks, 1)) * kBands, &d_edges));
     EPSEON_HIP_TRY(arena_array(a, nw, &ctx->d_win_full));
     EPSEON_HIP_TRY(arena_array(a, nw, &ctx->d_win_band));
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_brackets));
@@ -1128,12 +1148,13 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_nodes, 0, ne * sizeof(int32_t), ctx->stream));
     EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_far, 0, ne * sizeof(double), ctx->stream));
     EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_resc, 0, ne * sizeof(int32_t), ctx->stream));
-    EPSEON_HIP_TRY(launch_shift_potential(ctx->stream, v_src, ctx->d_rec, count, max_points,
-                                          ctx->d_ut, ctx->d_uv, ctx->d_uvr));
+    EPSEON_HIP_TRY(launch_shift_potential(ctx->stream, v_src, ctx->d_rec, count, max_table_chunks,
+                                          ctx->d_ut, ctx->d_uv, ctx->d_uvr, d_edges));
     // Band windows: computed on the device, read back to size the segment
     // tables and to give each window its far-end scale.
     std::vector<int2> raw(static_cast<size_t>(count) * kBands);
-    EPSEON_HIP_TRY(launch_band_windows(ctx->stream, ctx->d_uv, ctx->d_rec, count, d_raw_windows));
+    EPSEON_HIP_TRY(launch_band_windows(ctx->stream, ctx->d_uv, ctx->d_rec, count,
+                                       all_points / std::max(count, 1), d_edges, d_raw_windows));
     if (count > 0)
         EPSEON_HIP_TRY(hipMemcpyAsync(raw.data(), d_raw_windows, raw.size() * sizeof(int2),
                                       hipMemcpyDeviceToHost, ctx->stream));

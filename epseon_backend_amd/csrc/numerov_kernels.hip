@@ -468,103 +468,244 @@ __device__ __forceinline__ bool fetch_block_task(const WaveTask* __restrict__ ta
 
 }  // namespace
 
-// Statistics of each V table in device memory (one block per potential),
-// with the host loader's semantics: first index of the minimum, first
-// non-finite index, and the wall-trimmed Dirichlet points.
-__global__ __launch_bounds__(256) void potential_stats_kernel(const double* __restrict__ v,
-                                                              const int64_t* __restrict__ offsets,
-                                                              const int64_t* __restrict__ counts,
-                                                              const double* __restrict__ betas,
-                                                              PotentialStats* __restrict__ out)
+namespace {
+
+// Minimum, its first index and the first non-finite index (int64 max: none)
+// of the 256 threads' values, in every thread.  The value is reduced first;
+// the indices of the lanes that hold it follow.
+struct MinAt {
+    double v;
+    int64_t i, bad;
+};
+
+__device__ __forceinline__ int64_t wave_min64(int64_t x)
 {
-    __shared__ double s_v[256];
-    __shared__ int64_t s_i[256], s_b[256];
-    const int32_t p = static_cast<int32_t>(blockIdx.x);
-    const int32_t t = static_cast<int32_t>(threadIdx.x);
-    const double* base = v + offsets[p];
+#pragma unroll
+    for (int32_t d = 32; d >= 1; d /= 2) {
+        const int64_t o = __shfl_xor(x, d, 64);
+        x = o < x ? o : x;
+    }
+    return x;
+}
+
+__device__ __forceinline__ MinAt block_min(const MinAt& m)
+{
+    __shared__ double s_v[4];
+    __shared__ int64_t s_i[4], s_b[4];
+    double v = m.v;
+#pragma unroll
+    for (int32_t d = 32; d >= 1; d /= 2)
+        v = fmin(v, __shfl_xor(v, d, 64));
+    const int64_t i = wave_min64(m.v == v ? m.i : INT64_MAX);
+    const int64_t bad = __ballot(m.bad != INT64_MAX) != 0 ? wave_min64(m.bad) : INT64_MAX;
+    const int32_t w = static_cast<int32_t>(threadIdx.x >> 6);
+    if ((threadIdx.x & 63) == 0) {
+        s_v[w] = v;
+        s_i[w] = i;
+        s_b[w] = bad;
+    }
+    __syncthreads();
+    MinAt r{s_v[0], s_i[0], s_b[0]};
+#pragma unroll
+    for (int32_t q = 1; q < 4; ++q) {
+        if (s_v[q] < r.v || (s_v[q] == r.v && s_i[q] < r.i)) {
+            r.v = s_v[q];
+            r.i = s_i[q];
+        }
+        r.bad = s_b[q] < r.bad ? s_b[q] : r.bad;
+    }
+    return r;
+}
+
+}  // namespace
+
+// Statistics of each V table in device memory, with the host loader's
+// semantics: first index of the minimum, first non-finite index, and the
+// wall-trimmed Dirichlet points.  Two passes of one workgroup per chunk
+// (kStatsChunk points or more): the minimum of every chunk, then, from the
+// minimum of the potential's chunks, the walls.  Memory-bound from a few
+// hundred chunks on (256 x 50,000 points: 21 us a pass, 5 TB/s).  One workgroup
+// per potential with one load in flight per thread took 166 us there and
+// 2.89 ms for 1,000,000 points (now 8 and 5 us).
+__global__ __launch_bounds__(256) void potential_min_kernel(const double* __restrict__ v,
+                                                            const int64_t* __restrict__ offsets,
+                                                            const int64_t* __restrict__ counts,
+                                                            const int32_t* __restrict__ chunk0,
+                                                            ChunkMin* __restrict__ chunks,
+                                                            PotentialStats* __restrict__ out)
+{
+    const int32_t p = static_cast<int32_t>(blockIdx.y);
+    const int32_t c = static_cast<int32_t>(blockIdx.x);
     const int64_t n = counts[p];
-    double best = __builtin_inf();
-    int64_t bi = n, bad = n;
-    for (int64_t i = t; i < n; i += 256) {
-        const double x = base[i];
-        if (!__builtin_isfinite(x)) {
-            bad = i < bad ? i : bad;
-        } else if (x < best || (x == best && i < bi)) {
-            best = x;
-            bi = i;
-        }
-    }
-    s_v[t] = best;
-    s_i[t] = bi;
-    s_b[t] = bad;
-    __syncthreads();
-    for (int32_t d = 128; d > 0; d >>= 1) {
-        if (t < d) {
-            const double ov = s_v[t + d];
-            const int64_t oi = s_i[t + d];
-            if (ov < s_v[t] || (ov == s_v[t] && oi < s_i[t])) {
-                s_v[t] = ov;
-                s_i[t] = oi;
+    const int32_t len = load_chunk(n, kStatsChunk);
+    const int64_t i0 = static_cast<int64_t>(c) * len;
+    if (i0 >= n)
+        return;
+    const double* base = v + offsets[p];
+    const int64_t i1 = min(n, i0 + len);
+    MinAt m{__builtin_inf(), INT64_MAX, INT64_MAX};
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += 4 * 256) {
+        double x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            x[q] = base[min(i + 256 * q, i1 - 1)];
+        // Indices rise within a thread: a later equal value changes nothing.
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t at = min(i + 256 * q, i1 - 1);
+            if (!__builtin_isfinite(x[q])) {
+                m.bad = at < m.bad ? at : m.bad;
+            } else if (x[q] < m.v) {
+                m.v = x[q];
+                m.i = at;
             }
-            s_b[t] = s_b[t + d] < s_b[t] ? s_b[t + d] : s_b[t];
         }
-        __syncthreads();
     }
-    const double vmin = s_v[0];
-    const int64_t imin = s_i[0];
-    const int64_t first_bad = s_b[0];
-    __syncthreads();
+    m = block_min(m);
+    if (threadIdx.x == 0) {
+        chunks[chunk0[p] + c] = ChunkMin{m.v, m.i, m.bad};
+        if (c == 0)
+            out[p] = PotentialStats{0.0, 0, 0, n - 1, n};
+    }
+}
+
+__global__ __launch_bounds__(256) void potential_trim_kernel(const double* __restrict__ v,
+                                                             const int64_t* __restrict__ offsets,
+                                                             const int64_t* __restrict__ counts,
+                                                             const int32_t* __restrict__ chunk0,
+                                                             const double* __restrict__ betas,
+                                                             const ChunkMin* __restrict__ chunks,
+                                                             PotentialStats* __restrict__ out)
+{
+    const int32_t p = static_cast<int32_t>(blockIdx.y);
+    const int32_t c = static_cast<int32_t>(blockIdx.x);
+    const int64_t n = counts[p];
+    const int32_t len = load_chunk(n, kStatsChunk);
+    const int64_t i0 = static_cast<int64_t>(c) * len;
+    if (i0 >= n)
+        return;
+    const double* base = v + offsets[p];
+    const int64_t i1 = min(n, i0 + len);
+    const int32_t t = static_cast<int32_t>(threadIdx.x);
+    MinAt m{__builtin_inf(), INT64_MAX, INT64_MAX};
+    if (t < load_chunks(n, kStatsChunk)) {  // at most 256
+        const ChunkMin k = chunks[chunk0[p] + t];
+        m = MinAt{k.vmin, k.imin, k.bad};
+    }
+    m = block_min(m);
+    if (c == 0 && t == 0) {
+        out[p].vmin = m.i < n ? base[m.i] : m.v;
+        out[p].imin = min(m.i, n);
+        out[p].bad = min(m.bad, n);
+    }
     // Trimming needs a finite table with a minimum.
-    int64_t first = 0, last = n - 1;
-    if (first_bad == n && imin < n) {
-        const double wall = vmin + 0.5 / betas[p];
-        int64_t lo = -1, hi = n;
-        for (int64_t i = t; i <= imin; i += 256)
-            if (base[i] >= wall && i > lo)
-                lo = i;
-        for (int64_t i = imin + t; i < n; i += 256)
-            if (base[i] >= wall && i < hi)
-                hi = i;
-        s_i[t] = lo;
-        s_b[t] = hi;
-        __syncthreads();
-        for (int32_t d = 128; d > 0; d >>= 1) {
-            if (t < d) {
-                s_i[t] = s_i[t + d] > s_i[t] ? s_i[t + d] : s_i[t];
-                s_b[t] = s_b[t + d] < s_b[t] ? s_b[t + d] : s_b[t];
+    if (m.bad < n || m.i >= n)
+        return;
+    const double wall = m.v + 0.5 / betas[p];
+    int64_t lo = -1, hi = n;
+    for (int64_t i = i0 + t; i < i1; i += 4 * 256) {
+        double x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            x[q] = base[min(i + 256 * q, i1 - 1)];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t at = min(i + 256 * q, i1 - 1);
+            if (x[q] >= wall) {
+                if (at <= m.i && at > lo)
+                    lo = at;
+                if (at >= m.i && at < hi)
+                    hi = at;
             }
-            __syncthreads();
         }
-        if (s_i[0] >= 0)
-            first = s_i[0];
-        if (s_b[0] < n)
-            last = s_b[0];
     }
-    if (t == 0)
-        out[p] = PotentialStats{vmin, imin, first, last, first_bad};
+#pragma unroll
+    for (int32_t d = 32; d >= 1; d /= 2) {
+        const int64_t ol = __shfl_xor(lo, d, 64), oh = __shfl_xor(hi, d, 64);
+        lo = ol > lo ? ol : lo;
+        hi = oh < hi ? oh : hi;
+    }
+    // The previous pass left the grid ends, 0 and n - 1.
+    if ((t & 63) == 0) {
+        if (lo > 0)
+            atomicMax(reinterpret_cast<unsigned long long*>(&out[p].first), static_cast<unsigned long long>(lo));
+        if (hi < n - 1)
+            atomicMin(reinterpret_cast<unsigned long long*>(&out[p].last), static_cast<unsigned long long>(hi));
+    }
 }
 
 // p_i = fma(beta_p, V_i, -1) / 12 (scan table), uv_i = beta_p V_i (refinement
 // table) and the reversed refinement table uvr_i = uv_{n-1-i} (inward shots
 // from the right wall) for every point of the trimmed grid of every potential,
-// read from V in the caller's layout.
+// read from V in the caller's layout; and, from the same values, the first
+// and last allowed point (uv_i <= e_b) of every band top in the chunk.  One
+// workgroup of four wavefronts per chunk; a wavefront takes 64 consecutive
+// points at a time, so each band's edges are bit positions of a ballot.
+// Memory-bound (32 B per point).
 __global__ __launch_bounds__(256) void shift_potential_kernel(const double* __restrict__ v,
                                                               const PotentialRecord* __restrict__ pots,
                                                               double* __restrict__ ut,
                                                               double* __restrict__ uv,
-                                                              double* __restrict__ uvr)
+                                                              double* __restrict__ uvr,
+                                                              ChunkEdge* __restrict__ edges)
 {
+    __shared__ int32_t s_first[4][kBands], s_last[4][kBands];
     const PotentialRecord& P = pots[blockIdx.y];
-    const double beta = P.beta;
+    const int32_t len = load_chunk(P.full_points, kTableChunk);
+    const int32_t i0 = static_cast<int32_t>(blockIdx.x) * len;
     const int32_t n = P.n_points;
+    if (i0 >= P.full_points || P.flags != 0)  // rejected potentials are never shot
+        return;
+    const int32_t lane = static_cast<int32_t>(threadIdx.x & 63);
+    const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x >> 6));
+    const int32_t i1 = min(n, i0 + len);
+    const double beta = P.beta;
     const double* src = v + P.user_offset + P.first_point;
-    for (int32_t i = static_cast<int32_t>(blockIdx.x * blockDim.x + threadIdx.x); i < n;
-         i += static_cast<int32_t>(gridDim.x * blockDim.x)) {
-        const double x = src[i];
-        const double b = beta * x;
-        ut[P.ut_offset + i] = __builtin_fma(beta, x, -1.0) / 12.0;
-        uv[P.ut_offset + i] = b;
-        uvr[P.ut_offset + (n - 1 - i)] = b;
+    double eb[kBands];
+    int32_t first[kBands], last[kBands];
+#pragma unroll
+    for (int32_t b = 0; b < kBands; ++b) {
+        eb[b] = beta * __builtin_fma(static_cast<double>(b + 1), (P.e_hi - P.e_lo) / kBands, P.e_lo);
+        first[b] = n;
+        last[b] = -1;
+    }
+    for (int32_t base = i0 + 64 * wave; base < i1; base += 256) {
+        const int32_t i = base + lane;
+        const bool in = i < i1;
+        double u = __builtin_inf();
+        if (in) {
+            const double x = src[i];
+            u = beta * x;
+            ut[P.ut_offset + i] = __builtin_fma(beta, x, -1.0) / 12.0;
+            uv[P.ut_offset + i] = u;
+            uvr[P.ut_offset + (n - 1 - i)] = u;
+        }
+#pragma unroll
+        for (int32_t b = 0; b < kBands; ++b) {
+            const uint64_t mask = __ballot(in && u <= eb[b]);
+            if (mask != 0) {
+                first[b] = min(first[b], base + static_cast<int32_t>(__builtin_ctzll(mask)));
+                last[b] = base + 63 - static_cast<int32_t>(__builtin_clzll(mask));
+            }
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int32_t b = 0; b < kBands; ++b) {
+            s_first[wave][b] = first[b];
+            s_last[wave][b] = last[b];
+        }
+    }
+    __syncthreads();
+    const int32_t b = static_cast<int32_t>(threadIdx.x);
+    if (b < kBands) {
+        ChunkEdge e{n, -1};
+#pragma unroll
+        for (int32_t w = 0; w < 4; ++w) {
+            e.first = min(e.first, s_first[w][b]);
+            e.last = max(e.last, s_last[w][b]);
+        }
+        edges[(static_cast<int64_t>(P.chunk0) + blockIdx.x) * kBands + b] = e;
     }
 }
 
@@ -589,204 +730,167 @@ __device__ __forceinline__ bool same_window(const BandWindow* W, const int32_t a
     return W[a].lo == W[b].lo && W[a].hi == W[b].hi;
 }
 
-// floor(sqrt(n)) for n < 2^53 (the double square root, then corrected).
-__device__ __forceinline__ uint64_t isqrt_exact(const uint64_t n)
+// floor(sqrt(n)) of an integer n < 2^49 held in a double: the reciprocal
+// square root and one Newton step are within 1 of it, and the residual, exact
+// in a double (r < 2^25), settles which side.
+__device__ __forceinline__ double isqrt_exact(const double n)
 {
-    uint64_t r = static_cast<uint64_t>(__builtin_sqrt(static_cast<double>(n)));
-    while (r * r > n)
-        --r;
-    while ((r + 1) * (r + 1) <= n)
-        ++r;
+    const double y = __builtin_amdgcn_rsq(n);
+    const double s = n * y;
+    double r = floor(__builtin_fma(__builtin_fma(-s, s, n), 0.5 * y, s));
+    const double e = __builtin_fma(-r, r, n);
+    r = e < 0.0 ? r - 1.0 : (e > 2.0 * r ? r + 1.0 : r);
     return r;
 }
+
+// floor(65536 acosh(1 + y/2)/sqrt(y)) at y = 2^k, k = -5 .. 3.
+__device__ constexpr double kGrowthRatio[9] = {65450, 65366, 65199, 64871, 64242, 63073, 61029, 57761, 53116};
 
 // Lower bound g(x) of the per-step growth acosh(1 + x/2) in 2^-40 fixed
 // point, within 9 % of it: with x = m 2^k (m in [1/2, 1)) and T the top 16
 // bits of m's significand, x >= T 2^(k-16), and sqrt(T 2^(k-16)) 2^40 =
 // sqrt(T 2^r) 2^h (k + 64 = 2 h + r) is taken as isqrt(T 2^(r+32)) 2^(h-16),
-// floored, times floor(65536 acosh(1 + y/2)/sqrt(y)) at y = 2^k (the ratio
-// falls with y; entry -5 serves below) over 65536.  Integer operations only
-// after frexp.  0 below 2^-65; x >= 8 counts as just below 8.
-__device__ __forceinline__ int64_t growth_term(const double x)
+// floored, times the growth ratio at 2^k (the ratio falls with y; entry -5
+// serves below) over 65536.  Whole numbers held in doubles: T and k come from
+// the bits of x, every product has at most 41 significant bits and every sum
+// of terms stays below 2^53, so all of it is exact.  0 below 2^-65; x >= 8
+// counts as just below 8.  `ratio`: kGrowthRatio in LDS.  About 30
+// instructions where 64-bit integers took four times as many.
+__device__ __forceinline__ double growth_term(const double x, const double* ratio)
 {
-    constexpr int64_t kRatio[9] = {65450, 65366, 65199, 64871, 64242, 63073, 61029, 57761, 53116};
-    int k = 0;
-    const double m = __builtin_frexp(x, &k);
-    if (!(x > 0.0) || k < -64)
-        return 0;
-    uint64_t t = static_cast<uint64_t>(__builtin_ldexp(m, 16));
+    const uint32_t hi = static_cast<uint32_t>(static_cast<uint64_t>(__double_as_longlong(x)) >> 32);
+    int32_t k = static_cast<int32_t>((hi >> 20) & 0x7FFu) - 1022;
+    uint32_t t = 0x8000u | ((hi >> 5) & 0x7FFFu);
+    const bool counts = x > 0.0 && k >= -64;
     if (k > 3) {
         k = 3;
         t = 0xFFFF;
     }
+    k = max(k, -64);
     const int32_t e = k + 64, h = e >> 1;
-    const uint64_t r = isqrt_exact(t << ((e & 1) + 32));
-    const uint64_t sq = h >= 16 ? r << (h - 16) : r >> (16 - h);
-    int64_t f = kRatio[0];
-#pragma unroll
-    for (int32_t i = 1; i < 9; ++i)
-        if (k == i - 5)
-            f = kRatio[i];
-    return static_cast<int64_t>((sq * static_cast<uint64_t>(f)) >> 16);
+    const double r = isqrt_exact(__builtin_ldexp(static_cast<double>(t), (e & 1) + 32));
+    const double sq = floor(__builtin_ldexp(r, h - 16));
+    const double g = floor(__builtin_ldexp(sq * ratio[max(k, -5) + 5], -16));
+    return counts ? g : 0.0;
 }
 
-__device__ __forceinline__ int64_t wave_inclusive_sum(int64_t x)
+// Sum over the wavefront's lanes up to this one.
+__device__ __forceinline__ double wave_inclusive_sum(double x)
 {
     const int32_t lane = static_cast<int32_t>(threadIdx.x & 63);
 #pragma unroll
     for (int32_t d = 1; d < 64; d *= 2) {
-        const int64_t y = __shfl_up(x, d, 64);
+        const double y = __shfl_up(x, d, 64);
         if (lane >= d)
             x += y;
     }
     return x;
 }
 
-__device__ __forceinline__ int32_t wave_min(int32_t x)
-{
-#pragma unroll
-    for (int32_t d = 32; d >= 1; d /= 2)
-        x = min(x, __shfl_xor(x, d, 64));
-    return x;
-}
-
-__device__ __forceinline__ int32_t wave_max(int32_t x)
-{
-#pragma unroll
-    for (int32_t d = 32; d >= 1; d /= 2)
-        x = max(x, __shfl_xor(x, d, 64));
-    return x;
-}
-
 }  // namespace
 
-namespace {
-
-// Walk a fringe of the window at e from `start` by `dir` (+1: right, -1:
-// left), 64 points per step, until the depth sum reaches kWindowDepth;
-// returns the point where it does, or the grid end.  One wavefront.
-__device__ __forceinline__ int32_t fringe_end(const double* __restrict__ u, const int32_t n, const double e,
-                                              const int32_t start, const int32_t dir)
+// Band windows: one workgroup of W wavefronts per (potential, band, side).
+// The band's first and last allowed points come from the potential's chunks
+// (shift_potential_kernel); from there the workgroup walks the fringe, 512 W
+// points at a time, until the depth sum reaches kWindowDepth, and ends at the
+// point where it does, or at the grid end.  Writes lo or hi of the band (the
+// whole grid for rejected potentials).  Bound by the growth terms of the long
+// outer fringes.  One workgroup per potential for all of them: 1,000,000
+// points 3.56 ms (now 0.11), 8 x 200,000 points 1.33 ms (0.05), 256 x 50,000
+// points 0.52 ms (0.23), 10,000 points 84 us (8).
+template <int W>
+__global__ __launch_bounds__(64 * W) void band_window_kernel(const double* __restrict__ uv,
+                                                             const PotentialRecord* __restrict__ pots,
+                                                             const ChunkEdge* __restrict__ edges,
+                                                             int2* __restrict__ out)
 {
-    // Chunks of 64 x kPer points, kPer consecutive ones (in walk order) per
-    // lane: each lane sums its terms, one wave prefix sum orders the lanes,
-    // and the first lane reaching the depth finds the crossing among its own.
-    constexpr int32_t kPer = 8;
-    const int32_t lane = static_cast<int32_t>(threadIdx.x & 63);
-    const int64_t depth = int64_t(kWindowDepth) << 40;
-    int64_t acc = 0;
-    for (int32_t base = start; base >= 0 && base < n; base += 64 * kPer * dir) {
-        int64_t g[kPer];
-        int64_t own = 0;
-#pragma unroll
-        for (int32_t q = 0; q < kPer; ++q) {
-            const int32_t i = base + dir * (kPer * lane + q);
-            g[q] = (i >= 0 && i < n) ? growth_term(12.0 * (u[i] - e)) : 0;
-            own += g[q];
-        }
-        const int64_t inc = wave_inclusive_sum(own);
-        const uint64_t hit = __ballot(acc + inc >= depth);
-        if (hit != 0) {
-            const int32_t h = static_cast<int32_t>(__builtin_ctzll(hit));
-            int64_t run = acc + inc - own;
-            int32_t at = kPer - 1;
-            bool found = false;
-#pragma unroll
-            for (int32_t q = 0; q < kPer; ++q) {
-                run += g[q];
-                if (!found && run >= depth) {
-                    at = q;
-                    found = true;
-                }
-            }
-            return base + dir * (kPer * h + __shfl(at, h, 64));
-        }
-        acc += __shfl(inc, 63, 64);
-    }
-    return dir > 0 ? n - 1 : 0;
-}
-
-}  // namespace
-
-// Band windows: one workgroup of kBandWaves wavefronts per potential.  One
-// pass over the table finds the first and last allowed point (uv_i <= e_b)
-// of all kBands band tops at once; then the wavefronts walk the 2 kBands
-// fringes.  Writes (lo, hi) per band (whole grid for rejected potentials).
-constexpr int32_t kBandWaves = 16;
-__global__ __launch_bounds__(64 * kBandWaves) void band_window_kernel(const double* __restrict__ uv,
-                                                          const PotentialRecord* __restrict__ pots,
-                                                          const int32_t n_pots, int2* __restrict__ out)
-{
-    __shared__ int32_t s_first[kBandWaves][kBands], s_last[kBandWaves][kBands];
-    __shared__ int32_t s_win[2][kBands];
-    const int32_t p = static_cast<int32_t>(blockIdx.x);
-    if (p >= n_pots)
-        return;
+    constexpr int32_t kPer = 8, kT = 64 * W;
+    __shared__ double s_ratio[9];
+    __shared__ double s_sum[2][W];
+    __shared__ int32_t s_edge[W];
+    const int32_t p = static_cast<int32_t>(blockIdx.x) / (2 * kBands);
+    const int32_t b = static_cast<int32_t>(blockIdx.x) % (2 * kBands) >> 1;
+    const int32_t dir = (blockIdx.x & 1u) != 0 ? 1 : -1;
     const PotentialRecord& P = pots[p];
     const int32_t tid = static_cast<int32_t>(threadIdx.x);
     const int32_t lane = tid & 63, wave = tid >> 6;
     const int32_t n = P.n_points;
+    int32_t* end = dir > 0 ? &out[p * kBands + b].y : &out[p * kBands + b].x;
+    const int32_t grid_end = dir > 0 ? n - 1 : 0;
     if (P.flags != 0) {
-        if (tid < kBands)
-            out[p * kBands + tid] = make_int2(0, n - 1);
+        if (tid == 0)
+            *end = grid_end;
         return;
     }
+    if (tid < 9)
+        s_ratio[tid] = kGrowthRatio[tid];
+    // The outermost allowed point: n (left) or -1 (right) when there is none.
+    int32_t edge = dir > 0 ? -1 : n;
+    for (int32_t c = tid; c < load_chunks(P.full_points, kTableChunk); c += kT) {
+        const ChunkEdge k = edges[(static_cast<int64_t>(P.chunk0) + c) * kBands + b];
+        edge = dir > 0 ? max(edge, k.last) : min(edge, k.first);
+    }
+#pragma unroll
+    for (int32_t d = 32; d >= 1; d /= 2) {
+        const int32_t o = __shfl_xor(edge, d, 64);
+        edge = dir > 0 ? max(edge, o) : min(edge, o);
+    }
+    if (lane == 0)
+        s_edge[wave] = edge;
+    __syncthreads();
+#pragma unroll
+    for (int32_t w = 0; w < W; ++w)
+        edge = dir > 0 ? max(edge, s_edge[w]) : min(edge, s_edge[w]);
     const double* u = uv + P.ut_offset;
-    double eb[kBands];
-    int32_t first[kBands], last[kBands];
+    const double e = P.beta * __builtin_fma(static_cast<double>(b + 1), (P.e_hi - P.e_lo) / kBands, P.e_lo);
+    const double depth = static_cast<double>(int64_t(kWindowDepth) << 40);
+    double acc = 0.0;
+    // No allowed point: the grid end (its edge lies outside the grid).
+    const bool any = dir > 0 ? edge >= 0 : edge < n;
+    int32_t turn = 0;
+    for (int32_t base = edge + dir; any && base >= 0 && base < n; base += kT * kPer * dir, turn ^= 1) {
+        // kPer consecutive points per thread.
+        double g[kPer];
+        double own = 0.0;
 #pragma unroll
-    for (int32_t b = 0; b < kBands; ++b) {
-        eb[b] = P.beta * __builtin_fma(static_cast<double>(b + 1), (P.e_hi - P.e_lo) / kBands, P.e_lo);
-        first[b] = n;
-        last[b] = -1;
-    }
-    // Four loads in flight per thread.
-    constexpr int32_t kT = 64 * kBandWaves;
-    for (int32_t i0 = tid; i0 < n; i0 += 4 * kT) {
-        double x[4];
+        for (int32_t q = 0; q < kPer; ++q) {
+            const int32_t i = base + dir * (kPer * tid + q);
+            g[q] = (i >= 0 && i < n) ? growth_term(12.0 * (u[i] - e), s_ratio) : 0.0;
+            own += g[q];
+        }
+        const double inc = wave_inclusive_sum(own);
+        if (lane == 63)
+            s_sum[turn][wave] = inc;
+        __syncthreads();
+        double total = 0.0, before = 0.0;
 #pragma unroll
-        for (int32_t q = 0; q < 4; ++q)
-            x[q] = i0 + q * kT < n ? u[i0 + q * kT] : __builtin_inf();
+        for (int32_t w = 0; w < W; ++w) {
+            before += w < wave ? s_sum[turn][w] : 0.0;
+            total += s_sum[turn][w];
+        }
+        if (acc + total < depth) {
+            acc += total;
+            continue;
+        }
+        double run = acc + before + (inc - own);
+        // Exactly one thread's points take the sum from below the depth to it.
+        if (run < depth && run + own >= depth) {
+            int32_t at = kPer - 1;
+            bool hit = false;
 #pragma unroll
-        for (int32_t q = 0; q < 4; ++q)
-#pragma unroll
-            for (int32_t b = 0; b < kBands; ++b)
-                if (x[q] <= eb[b]) {
-                    first[b] = min(first[b], i0 + q * kT);
-                    last[b] = i0 + q * kT;
+            for (int32_t q = 0; q < kPer; ++q) {
+                run += g[q];
+                if (!hit && run >= depth) {
+                    at = q;
+                    hit = true;
                 }
-    }
-#pragma unroll
-    for (int32_t b = 0; b < kBands; ++b) {
-        first[b] = wave_min(first[b]);
-        last[b] = wave_max(last[b]);
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int32_t b = 0; b < kBands; ++b) {
-            s_first[wave][b] = first[b];
-            s_last[wave][b] = last[b];
+            }
+            *end = base + dir * (kPer * tid + at);
         }
+        return;
     }
-    __syncthreads();
-    // Fringe walks: task t = 2 b + side, wavefront w takes t = w, w + kBandWaves, ...
-    for (int32_t t = wave; t < 2 * kBands; t += kBandWaves) {
-        const int32_t b = t >> 1, side = t & 1;
-        int32_t f = s_first[0][b], l = s_last[0][b];
-#pragma unroll
-        for (int32_t w = 1; w < kBandWaves; ++w) {
-            f = min(f, s_first[w][b]);
-            l = max(l, s_last[w][b]);
-        }
-        int32_t r = side ? n - 1 : 0;
-        if (l >= 0)
-            r = side ? fringe_end(u, n, eb[b], l + 1, 1) : fringe_end(u, n, eb[b], f - 1, -1);
-        if (lane == 0)
-            s_win[side][b] = r;
-    }
-    __syncthreads();
-    if (tid < kBands)
-        out[p * kBands + tid] = make_int2(s_win[0][tid], s_win[1][tid]);
+    if (tid == 0)
+        *end = grid_end;
 }
 
 // Scan: lane = trial energy E_j = fma(j+1, dE, E_lo) shot over the band
@@ -2375,27 +2479,37 @@ __global__ __launch_bounds__(256) void bracket_kernel(const PotentialRecord* __r
 
 // ---------------------------------------------------------------- launchers
 
+// chunk0[p]: the number of chunks of the potentials before p; max_chunks: the
+// most of one potential.
 hipError_t launch_potential_stats(hipStream_t stream, const double* v, const int64_t* offsets,
-                                  const int64_t* counts, const double* betas, int32_t n_pots,
-                                  PotentialStats* out)
+                                  const int64_t* counts, const int32_t* chunk0, const double* betas,
+                                  int32_t n_pots, int32_t max_chunks, ChunkMin* chunks, PotentialStats* out)
 {
-    if (n_pots == 0)
-        return hipSuccess;
-    hipLaunchKernelGGL(potential_stats_kernel, dim3(static_cast<unsigned>(n_pots)), dim3(256), 0, stream, v,
-                       offsets, counts, betas, out);
-    return hipGetLastError();
+    for (int32_t p = 0; p < n_pots; p += 65535) {
+        const dim3 grid(static_cast<unsigned>(max_chunks), static_cast<unsigned>(n_pots - p < 65535 ? n_pots - p : 65535));
+        hipLaunchKernelGGL(potential_min_kernel, grid, dim3(256), 0, stream, v, offsets + p, counts + p, chunk0 + p,
+                           chunks, out + p);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess)
+            return e;
+        hipLaunchKernelGGL(potential_trim_kernel, grid, dim3(256), 0, stream, v, offsets + p, counts + p, chunk0 + p,
+                           betas + p, chunks, out + p);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_shift_potential(hipStream_t stream, const double* v, const PotentialRecord* pots,
-                                  int32_t n_pots, int32_t max_points, double* ut, double* uv,
-                                  double* uvr)
+                                  int32_t n_pots, int32_t max_chunks, double* ut, double* uv,
+                                  double* uvr, ChunkEdge* edges)
 {
-    if (n_pots == 0)
-        return hipSuccess;
-    const int32_t bx = (max_points + 255) / 256;
-    dim3 grid(static_cast<unsigned>(bx < 1024 ? bx : 1024), static_cast<unsigned>(n_pots));
-    hipLaunchKernelGGL(shift_potential_kernel, grid, dim3(256), 0, stream, v, pots, ut, uv, uvr);
-    return hipGetLastError();
+    for (int32_t p = 0; p < n_pots; p += 65535) {
+        const dim3 grid(static_cast<unsigned>(max_chunks), static_cast<unsigned>(n_pots - p < 65535 ? n_pots - p : 65535));
+        hipLaunchKernelGGL(shift_potential_kernel, grid, dim3(256), 0, stream, v, pots + p, ut, uv, uvr, edges);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
 }
 
 // bins == nullptr: tasks[0, n_tasks) in order.  Otherwise `bins` (device, 9
@@ -2568,13 +2682,24 @@ hipError_t launch_level_summary(hipStream_t stream, const PotentialRecord* pots,
     return hipGetLastError();
 }
 
+// Wavefronts per fringe, mean_points being the potentials' mean size.  Below
+// 64 potentials the 32 fringes each leave the chip idle and a long fringe's
+// steps set the time: sixteen (8 x 200,000 points: 50 us; four: 99, one: 340).
+// From there the walk step of 512 points per wavefront should not overshoot
+// the fringes: four (256 x 50,000 points: 226 us; one: 288, sixteen: 358), and
+// one for short tables (1024 x 2,000 points: 56 us; two: 84, four: 139).
 hipError_t launch_band_windows(hipStream_t stream, const double* uv, const PotentialRecord* pots,
-                               int32_t n_pots, int2* out)
+                               int32_t n_pots, int64_t mean_points, const ChunkEdge* edges, int2* out)
 {
     if (n_pots == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(band_window_kernel, dim3(static_cast<unsigned>(n_pots)), dim3(64 * kBandWaves), 0, stream,
-                       uv, pots, n_pots, out);
+    const dim3 grid(static_cast<unsigned>(n_pots) * 2 * kBands);
+    if (n_pots < 64)
+        hipLaunchKernelGGL(band_window_kernel<16>, grid, dim3(1024), 0, stream, uv, pots, edges, out);
+    else if (mean_points >= 8192)
+        hipLaunchKernelGGL(band_window_kernel<4>, grid, dim3(256), 0, stream, uv, pots, edges, out);
+    else
+        hipLaunchKernelGGL(band_window_kernel<1>, grid, dim3(64), 0, stream, uv, pots, edges, out);
     return hipGetLastError();
 }
 

@@ -57,9 +57,40 @@ struct alignas(16) PotentialRecord {
     int32_t psi_seg_len;    // steps per segment of the eigenfunction shots (a multiple of 32)
     int32_t psi_segs_left;  // segments of the left shot (match steps)
     int32_t psi_segs_right; // segments of the right shot (n_points - 2 - match steps)
-    int32_t psi_pad;
+    int32_t chunk0;         // first chunk of this potential in the table pass's edge array
 };
 static_assert(sizeof(PotentialRecord) == 176, "record layout");
+
+// The load passes split a potential's n_points (untrimmed) values into chunks,
+// one workgroup each: the table pass takes 1024 points, the statistics passes
+// 4096 (their reduction costs as much as a few thousand loads), or more so
+// that there are at most 256 chunks.
+constexpr int32_t kTableChunk = 1024, kStatsChunk = 4096;
+
+constexpr int32_t load_chunk(const int64_t n_points, const int32_t least)
+{
+    const int64_t c = ((n_points + 255) / 256 + 255) & ~int64_t(255);
+    return static_cast<int32_t>(c < least ? least : c);
+}
+
+constexpr int32_t load_chunks(const int64_t n_points, const int32_t least)
+{
+    const int32_t c = load_chunk(n_points, least);
+    return static_cast<int32_t>((n_points + c - 1) / c);
+}
+
+// Minimum of one chunk of a V table: value, first index (n_points if the
+// chunk has no finite value) and first non-finite index (n_points if none).
+struct ChunkMin {
+    double vmin;
+    int64_t imin, bad;
+};
+
+// First and last allowed point of one band in one chunk of a trimmed table
+// (n_points and -1 when there is none).
+struct ChunkEdge {
+    int32_t first, last;
+};
 
 // Segments of the 64-lane segmented refinement of a potential with n points:
 // the q = n - 2 steps split into min(64, max(1, q / 32)) segments, segment s
