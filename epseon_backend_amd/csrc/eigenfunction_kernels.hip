@@ -418,69 +418,108 @@ __global__ __launch_bounds__(64) void psi_segment_kernel(
         PsiSegMatrix{B.ay, B.aym, B.ad, B.by, B.bym, B.bd, B.saa, B.sab, B.sbb, B.ex, 0};
 }
 
-// Pass 1b: one lane per level (wavefront = up to 64 levels of one potential).
-// Chains the segment matrices of each side from its wall, (y, y_prev, d) =
-// (1, 0, 1), renormalising by a power of two after each product; writes the
-// checkpoint (state and binary exponent) at each later segment start, sums
-// y^2 as the segments' quadratic forms, matches the sides at m and writes the
-// level's LevelNorm (exponents in bits).
-__global__ __launch_bounds__(64) void normalize_kernel(
+// End state of one side's chained shot.
+struct SideEnd {
+    double y, ym, sum;
+    int32_t k;
+};
+
+// One side's shot, chained segment by segment.
+struct SideChain {
+    double y, ym, d, sum;
+    int32_t k;
+    __device__ __forceinline__ PsiCheckpoint state() const { return PsiCheckpoint{y, ym, d, k, 0}; }
+    __device__ __forceinline__ void append(const PsiSegMatrix& M)
+    {
+        const double g = __builtin_fma(y * y, M.saa, __builtin_fma(2.0 * y * d, M.sab, d * d * M.sbb));
+        const double yn = __builtin_fma(M.ay, y, M.by * d);
+        const double ymn = __builtin_fma(M.aym, y, M.bym * d);
+        const double dn = __builtin_fma(M.ad, y, M.bd * d);
+        const int32_t x = binary_exponent(fmax(fmax(fabs(yn), fabs(ymn)), fabs(dn)));
+        y = __builtin_ldexp(yn, -x);
+        ym = __builtin_ldexp(ymn, -x);
+        d = __builtin_ldexp(dn, -x);
+        // y^2 sum relative to 2^(2k) of the new exponent k + e + x.
+        sum = __builtin_ldexp(sum, -2 * (M.e + x)) + __builtin_ldexp(g, -2 * x);
+        k += M.e + x;
+    }
+};
+
+// Pass 1b: two wavefronts per 64 levels of one potential, one lane per level
+// and side.  Chains the segment matrices of the side from its wall,
+// (y, y_prev, d) = (1, 0, 1), renormalising by a power of two after each
+// product, and writes the checkpoint (state and binary exponent) at each later
+// segment start and the sum of y^2 as the segments' quadratic forms; then the
+// sides meet at m and the first wavefront writes the levels' LevelNorm
+// (exponents in bits).  Bound by the chain's latency: the matrices are loaded
+// kAhead segments before their use, which leaves about 15 dependent FP64
+// operations per segment.
+__global__ __launch_bounds__(128) void normalize_kernel(
     const PotentialRecord* __restrict__ pots, const WaveTask* __restrict__ tasks, const int32_t n_tasks,
     const int32_t* __restrict__ status, const PsiSegMatrix* __restrict__ mats,
     PsiCheckpoint* __restrict__ ckpt, LevelNorm* __restrict__ norms)
 {
+    constexpr int32_t kAhead = 4;
+    __shared__ SideEnd s_right[64];
     const int32_t tid = static_cast<int32_t>(blockIdx.x);
     if (tid >= n_tasks)
         return;
     const WaveTask task = tasks[tid];
     const PotentialRecord& P = pots[task.potential];
-    const int32_t l = task.first + static_cast<int32_t>(threadIdx.x);
-    if (l >= P.level_count)
-        return;
+    const int32_t lane = static_cast<int32_t>(threadIdx.x & 63);
+    const int32_t side = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x >> 6));
+    const int32_t l = task.first + lane;
     const int64_t o = P.level_offset + l;
-    if (P.flags != 0 || !level_active(status, o)) {
+    const bool valid = l < P.level_count;
+    const bool active = valid && P.flags == 0 && level_active(status, o);
+    SideEnd end{1.0, 0.0, 0.0, 0};
+    if (active) {
+        const int32_t segs = side == 0 ? P.psi_segs_left : P.psi_segs_right;
+        const int64_t stride = P.level_count;
+        const int64_t slot0 = psi_slot(P, side, 0, l);
+        SideChain c{1.0, 0.0, 1.0, 0.0, 0};
+        PsiSegMatrix next[kAhead];
+#pragma unroll
+        for (int32_t q = 0; q < kAhead; ++q)
+            next[q] = mats[slot0 + min(q, segs - 1) * stride];
+        int32_t sg = 0;
+        // The first segment's checkpoint (the wall) is written like the
+        // others and never read.
+        for (; sg + kAhead <= segs; sg += kAhead) {
+#pragma unroll
+            for (int32_t q = 0; q < kAhead; ++q) {
+                ckpt[slot0 + (sg + q) * stride] = c.state();
+                c.append(next[q]);
+                next[q] = mats[slot0 + min(sg + q + kAhead, segs - 1) * stride];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int32_t q = 0; q < kAhead - 1; ++q)
+            if (sg + q < segs) {
+                ckpt[slot0 + (sg + q) * stride] = c.state();
+                c.append(next[q]);
+            }
+        end = SideEnd{c.y, c.ym, c.sum, c.k};
+    }
+    if (side == 1)
+        s_right[lane] = end;
+    __syncthreads();
+    if (side == 1 || !valid)
+        return;
+    if (!active) {
         norms[o] = LevelNorm{0.0, 0.0, 0, 0};
         return;
     }
-    double ye[2], yme[2], srel[2];
-    int32_t ke[2];
-    for (int32_t side = 0; side < 2; ++side) {
-        const int32_t segs = side == 0 ? P.psi_segs_left : P.psi_segs_right;
-        double y = 1.0, ym = 0.0, d = 1.0, sr = 0.0;
-        int32_t k = 0;
-        for (int32_t sg = 0; sg < segs; ++sg) {
-            const int64_t slot = psi_slot(P, side, sg, l);
-            if (sg > 0)
-                ckpt[slot] = PsiCheckpoint{y, ym, d, k, 0};
-            const PsiSegMatrix M = mats[slot];
-            const double q = __builtin_fma(y * y, M.saa, __builtin_fma(2.0 * y * d, M.sab, d * d * M.sbb));
-            const double yn = __builtin_fma(M.ay, y, M.by * d);
-            const double ymn = __builtin_fma(M.aym, y, M.bym * d);
-            const double dn = __builtin_fma(M.ad, y, M.bd * d);
-            const double mx = fmax(fmax(fabs(yn), fabs(ymn)), fabs(dn));
-            const int32_t x = binary_exponent(mx);
-            y = __builtin_ldexp(yn, -x);
-            ym = __builtin_ldexp(ymn, -x);
-            d = __builtin_ldexp(dn, -x);
-            // y^2 sum relative to 2^(2k) of the new exponent k + e + x.
-            sr = __builtin_ldexp(sr, -2 * (M.e + x)) + __builtin_ldexp(q, -2 * x);
-            k += M.e + x;
-        }
-        ye[side] = y;
-        yme[side] = ym;
-        srel[side] = sr;
-        ke[side] = k;
-    }
+    const SideEnd right = s_right[lane];
     // Left: (y_m, y_{m+1}) = (ym, y); right (reversed): (y_{m+1}, y_m) = (ym, y);
     // the right shot scaled by c = cm 2^(k_left - k_right).
-    const double yl0 = yme[0], yl1 = ye[0];
-    const double yr1 = yme[1], yr0 = ye[1];
-    const double num = __builtin_fma(yl0, yr0, yl1 * yr1);
-    const double den = __builtin_fma(yr0, yr0, yr1 * yr1);
+    const double num = __builtin_fma(end.ym, right.y, end.y * right.ym);
+    const double den = __builtin_fma(right.y, right.y, right.ym * right.ym);
     const double cm = num / den;
-    const double s = __builtin_fma(cm * cm, srel[1], srel[0]);
+    const double s = __builtin_fma(cm * cm, right.sum, end.sum);
     const double a = 1.0 / sqrt(s * P.h);
-    norms[o] = LevelNorm{a, cm * a, ke[0], ke[1]};
+    norms[o] = LevelNorm{a, cm * a, end.k, right.k};
 }
 
 // Eigenfunctions: for each task (potential, first level, side, segment), the
@@ -640,7 +679,7 @@ hipError_t launch_normalize(hipStream_t stream, const double* uv, const double* 
     }
     if (n_tasks == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(normalize_kernel, dim3(static_cast<unsigned>(n_tasks)), dim3(64), 0, stream, pots, tasks,
+    hipLaunchKernelGGL(normalize_kernel, dim3(static_cast<unsigned>(n_tasks)), dim3(128), 0, stream, pots, tasks,
                        n_tasks, status, mats, ckpt, norms);
     return hipGetLastError();
 }

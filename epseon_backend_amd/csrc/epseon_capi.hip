@@ -834,7 +834,7 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         EPSEON_HIP_TRY(hipStreamSynchronize(ctx->stream));
     }
 
-    int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0;
+    int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0, psi_waves = 0;
     int32_t max_seg_rows = 0;
     double scan_pu = 0.0;
     for (int32_t p = 0; p < count; ++p) {
@@ -891,16 +891,12 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         max_seg_rows = std::max(max_seg_rows, seg_rows(r.n_points, r.flags, r.level_count));
         if (seg_total > INT32_MAX)
             return fail(EPSEON_ERR_INVALID, "batch too large for the segment table");
-        // Eigenfunction shots run in segments of psi_seg_len steps; the
-        // normalisation pass leaves a checkpoint per level at each segment
-        // start (slot 0 of each side is unused).
         r.psi_seg_len = psi_seg_len(r.n_points);
-        r.psi_segs_left = (r.match + r.psi_seg_len - 1) / r.psi_seg_len;
-        r.psi_segs_right = (r.n_points - 2 - r.match + r.psi_seg_len - 1) / r.psi_seg_len;
-        r.psi_ckpt = ckpt_total;
-        r.chunk0 = table_chunk0[static_cast<size_t>(p)];
         if (r.flags == EPSEON_POT_OK)
-            ckpt_total += static_cast<int64_t>(d.level_count) * (r.psi_segs_left + r.psi_segs_right);
+            psi_waves += static_cast<int64_t>((d.level_count + 63) / 64) *
+                         ((r.match + r.psi_seg_len - 1) / r.psi_seg_len +
+                          (r.n_points - 2 - r.match + r.psi_seg_len - 1) / r.psi_seg_len);
+        r.chunk0 = table_chunk0[static_cast<size_t>(p)];
         r.user_offset = v_offsets[p];
         r.psi_offset = psi_total;
         psi_total += static_cast<int64_t>(d.level_count) * d.n_points;
@@ -915,6 +911,18 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         lv += d.level_count;
         if (r.flags == EPSEON_POT_OK)
             scan_pu += static_cast<double>(r.n_points - 2) * static_cast<double>(d.n_energies);
+    }
+    // Eigenfunction shots run in segments of psi_seg_len steps; the
+    // normalisation pass leaves a checkpoint per level at each segment start
+    // (slot 0 of each side is unused).
+    for (PotentialRecord& r : ctx->rec) {
+        if (psi_waves < kPsiFewWaves)
+            r.psi_seg_len = psi_short_seg_len(r.n_points);
+        r.psi_segs_left = (r.match + r.psi_seg_len - 1) / r.psi_seg_len;
+        r.psi_segs_right = (r.n_points - 2 - r.match + r.psi_seg_len - 1) / r.psi_seg_len;
+        r.psi_ckpt = ckpt_total;
+        if (r.flags == EPSEON_POT_OK)
+            ckpt_total += static_cast<int64_t>(r.level_count) * (r.psi_segs_left + r.psi_segs_right);
     }
     ctx->total_points = pts;
     ctx->total_energies = en;

@@ -124,6 +124,23 @@ constexpr int32_t psi_seg_len(const int32_t n_points)
     return 32 * (blocks < 16 ? 16 : blocks);
 }
 
+// Batches whose segments at that length give fewer wavefronts than this (one
+// per SIMD) leave the chip idle while each pass walks a whole segment; their
+// segments are shortened.  The walk costs about 0.08 us per step (both passes)
+// and the normalisation's chain 0.14 us per segment of a side, so the sum is
+// least near 1.3 sqrt(n) steps: a multiple of 32, at least 64 and at most
+// psi_seg_len.
+constexpr int64_t kPsiFewWaves = 1024;
+constexpr int32_t psi_short_seg_len(const int32_t n_points)
+{
+    // 32 b >= 1.3 sqrt(n): b^2 >= 1.69 n / 1024.
+    int32_t b = 2;
+    while (static_cast<int64_t>(b) * b * 1024 * 100 < static_cast<int64_t>(169) * n_points)
+        ++b;
+    const int32_t most = psi_seg_len(n_points);
+    return 32 * b < most ? 32 * b : most;
+}
+
 // State of an eigenfunction shot at the start of one of its segments (after
 // j = segment * psi_seg_len steps): y_{j+1}, y_j and their difference as
 // mantissas of the binary exponent k (the true values are these times 2^k).
