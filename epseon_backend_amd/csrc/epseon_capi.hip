@@ -43,7 +43,7 @@ hipError_t launch_refine_segmented(hipStream_t, int32_t, int32_t, const double*,
                                    const int32_t*, int32_t, const Bracket*, RefinePoints*, double, int32_t,
                                    double*, int32_t*, int32_t*, int32_t*);
 hipError_t launch_segment_tables(hipStream_t, const double*, const PotentialRecord*, const TableJob*,
-                                 int32_t, int32_t, double*);
+                                 int32_t, int32_t, int32_t, double*);
 hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord*, int32_t, int64_t,
                                const ChunkEdge*, int2*);
 hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, int32_t, const int32_t*, const int32_t*,
@@ -169,6 +169,14 @@ constexpr int64_t kLanePerLevelMinLevels = int64_t(64) * 2048;
 // (two blocks per SIMD, with several rounds of blocks to balance the XCD bins).
 constexpr int64_t kPairMinLevelsPerCu = 24;
 constexpr int64_t kQuadMinLevelsPerCu = 96;
+
+// Batches that refine in blocks of 128 or 256 lanes get segment tables from
+// this many points on.  Measured per refinement, natural table against segment
+// table: 20 x 17 levels in 256 lanes, 10,000 points 48 and 46 us, 20,000 61 and
+// 55, 80,000 140 and 98; 115 levels of one potential, 10,000 points 67 and 65,
+// 160,000 184 and 140; 8 x 80 levels in 128 lanes, 20,000 points 60 and 54.
+// Below, the pass that builds them costs what they save.
+constexpr int32_t kWideTableMinPoints = 16384;
 
 // Automatic windows need at least this many scan wavefronts per SIMD.
 constexpr int64_t kWindowsMinScanWavesPerSimd = 8;
@@ -303,6 +311,12 @@ struct epseon_ctx {
     TableJob* d_table_jobs = nullptr;
     int32_t n_jobs_full = 0, n_jobs_band = 0, table_max_rows = 0;
     bool tables_full = false, tables_band = false;
+    // Segment tables of the wider blocks (128 or 256 lanes) that small batches
+    // refine in: built at load for the block width and window set of the
+    // tuning then in force; refinements with others read the natural table.
+    double* d_segtab_wide = nullptr;
+    int32_t wide_lanes = 0;  // 0: none
+    bool wide_band = false;
     int32_t* d_steps = nullptr;  // recurrence steps of each level's shots (its window's n - 2)
     Bracket* d_brackets = nullptr;  // each level's bracket from the last scan
     RefinePoints* d_points = nullptr;  // each level's interpolation points (bracket pass, refinement)
@@ -608,9 +622,9 @@ hipError_t build_tables(epseon_ctx* ctx, hipStream_t stream, bool band)
     built = true;
     if (band)
         return launch_segment_tables(stream, ctx->d_uv, ctx->d_rec, ctx->d_table_jobs + ctx->n_jobs_full,
-                                     ctx->n_jobs_band, ctx->table_max_rows, ctx->d_segtab_band);
+                                     ctx->n_jobs_band, ctx->table_max_rows, 64, ctx->d_segtab_band);
     return launch_segment_tables(stream, ctx->d_uv, ctx->d_rec, ctx->d_table_jobs, ctx->n_jobs_full,
-                                 ctx->table_max_rows, ctx->d_segtab_full);
+                                 ctx->table_max_rows, 64, ctx->d_segtab_full);
 }
 
 // Shared body of epseon_load_potentials (v_host) and
@@ -835,7 +849,7 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     }
 
     int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0, psi_waves = 0;
-    int32_t max_seg_rows = 0;
+    int32_t max_seg_rows = 0, longest = 0;
     double scan_pu = 0.0;
     for (int32_t p = 0; p < count; ++p) {
         const epseon_potential_desc& d = desc[p];
@@ -888,6 +902,7 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         }
         r.seg_row = static_cast<int32_t>(seg_total);
         seg_total += seg_rows(r.n_points, r.flags, r.level_count);
+        longest = std::max(longest, r.n_points);
         max_seg_rows = std::max(max_seg_rows, seg_rows(r.n_points, r.flags, r.level_count));
         if (seg_total > INT32_MAX)
             return fail(EPSEON_ERR_INVALID, "batch too large for the segment table");
@@ -1179,8 +1194,8 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
             jobs_full.push_back({p, 0, r.n_points, r.seg_row});
         for (int32_t b = 0; b < kBands; ++b) {
             const size_t i = static_cast<size_t>(p) * kBands + static_cast<size_t>(b);
-            win_full[i] = BandWindow{0, r.n_points - 1, r.far_exp, r.seg_row, r.far_scale};
-            BandWindow w{raw[i].x, raw[i].y, 0, 0, 1.0};
+            win_full[i] = BandWindow{0, r.n_points - 1, r.far_exp, r.seg_row, r.far_scale, 0, 0};
+            BandWindow w{raw[i].x, raw[i].y, 0, 0, 1.0, 0, 0};
             const int32_t n = w.hi - w.lo + 1;
             const double l2 = static_cast<double>(n - 2) * std::log2(12.0);
             const double fl = std::floor(l2);
@@ -1198,6 +1213,48 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
             }
             win_band[i] = w;
         }
+    }
+    // Tables for blocks wider than 64 lanes (small batches), of the window set
+    // that the current tuning's solve will use.
+    std::vector<TableJob> jobs_wide;
+    int32_t wide_max_rows = 0;
+    const int32_t mode_now = choose_refine_mode(ctx);
+    const int32_t lanes_now = segmented_lanes(ctx);
+    ctx->wide_lanes = 0;
+    if (mode_now == EPSEON_REFINE_SEGMENTED && lanes_now > 64 && longest >= kWideTableMinPoints) {
+        ctx->wide_band = windows_for(ctx, mode_now);
+        std::vector<BandWindow>& set = ctx->wide_band ? win_band : win_full;
+        int64_t rows = 0;
+        for (size_t i = 0; i < set.size(); ++i) {
+            const int32_t p = static_cast<int32_t>(i / kBands);
+            const PotentialRecord& r = ctx->rec[static_cast<size_t>(p)];
+            BandWindow& w = set[i];
+            const int32_t n = w.hi - w.lo + 1;
+            const int32_t need = seg_rows(n, r.flags, r.level_count, lanes_now);
+            if (need == 0)
+                continue;
+            if (i % kBands != 0 && set[i - 1].lo == w.lo && set[i - 1].hi == w.hi) {
+                w.wide_row = set[i - 1].wide_row;
+                continue;
+            }
+            w.wide_row = static_cast<int32_t>(rows);
+            jobs_wide.push_back({p, w.lo, n, w.wide_row});
+            rows += need;
+            wide_max_rows = std::max(wide_max_rows, need);
+            if (rows > INT32_MAX)
+                break;
+        }
+        // One table is read through a 32-bit-addressed buffer.  Without room
+        // the refinement reads the natural table.
+        if (!jobs_wide.empty() && rows <= INT32_MAX && wide_max_rows <= INT32_MAX / (8 * lanes_now)) {
+            if (arena_array(a, static_cast<size_t>(rows) * static_cast<size_t>(lanes_now), &ctx->d_segtab_wide) ==
+                hipSuccess)
+                ctx->wide_lanes = lanes_now;
+            else
+                (void)hipGetLastError();
+        }
+        if (ctx->wide_lanes == 0)
+            jobs_wide.clear();
     }
     // Windowed scan: work per task (trial energies times its band window's
     // steps), its total, and its own XCD bins with the longest tasks first.
@@ -1227,7 +1284,11 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     ctx->segtab_ok = max_rows <= INT32_MAX / 512;
     EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(band_total, 1)) * 64, &ctx->d_segtab_band));
     TableJob* d_jobs = nullptr;
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(jobs_full.size() + jobs_band.size(), 1), &d_jobs));
+    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(jobs_full.size() + jobs_band.size() + jobs_wide.size(), 1), &d_jobs));
+    TableJob* d_jobs_wide = d_jobs + jobs_full.size() + jobs_band.size();
+    if (!jobs_wide.empty())
+        EPSEON_HIP_TRY(hipMemcpyAsync(d_jobs_wide, jobs_wide.data(), jobs_wide.size() * sizeof(TableJob),
+                                      hipMemcpyHostToDevice, ctx->stream));
     ctx->d_table_jobs = d_jobs;
     ctx->n_jobs_full = static_cast<int32_t>(jobs_full.size());
     ctx->n_jobs_band = static_cast<int32_t>(jobs_band.size());
@@ -1246,17 +1307,20 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         EPSEON_HIP_TRY(hipMemcpyAsync(d_jobs + jobs_full.size(), jobs_band.data(),
                                       jobs_band.size() * sizeof(TableJob), hipMemcpyHostToDevice,
                                       ctx->stream));
-    if (ctx->segtab_ok && jobs_full.size() + jobs_band.size() > 0) {
-        // The set the current tuning's solve will use, built on stream2 while
-        // the next scan runs; the refinement waits for it (tables_pending).
-        const int32_t mode = choose_refine_mode(ctx);
-        if (mode == EPSEON_REFINE_SEGMENTED && segmented_lanes(ctx) == 64) {
-            EPSEON_HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
-            EPSEON_HIP_TRY(hipStreamWaitEvent(ctx->stream2, ctx->ev_fork, 0));
-            EPSEON_HIP_TRY(build_tables(ctx, ctx->stream2, windows_for(ctx, mode)));
-            EPSEON_HIP_TRY(hipEventRecord(ctx->ev_tables, ctx->stream2));
-            ctx->tables_pending = true;
-        }
+    // The tables the current tuning's solve will use, built on stream2 while
+    // the next scan runs; the refinement waits for them (tables_pending).
+    const bool build_64 = mode_now == EPSEON_REFINE_SEGMENTED && lanes_now == 64 && ctx->segtab_ok &&
+                          jobs_full.size() + jobs_band.size() > 0;
+    if (build_64 || !jobs_wide.empty()) {
+        EPSEON_HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
+        EPSEON_HIP_TRY(hipStreamWaitEvent(ctx->stream2, ctx->ev_fork, 0));
+        if (build_64)
+            EPSEON_HIP_TRY(build_tables(ctx, ctx->stream2, windows_for(ctx, mode_now)));
+        EPSEON_HIP_TRY(launch_segment_tables(ctx->stream2, ctx->d_uv, ctx->d_rec, d_jobs_wide,
+                                             static_cast<int32_t>(jobs_wide.size()), wide_max_rows,
+                                             lanes_now, ctx->d_segtab_wide));
+        EPSEON_HIP_TRY(hipEventRecord(ctx->ev_tables, ctx->stream2));
+        ctx->tables_pending = true;
     }
     // The host buffers are pageable and owned by the caller: finish the
     // copies before returning.
@@ -1461,8 +1525,11 @@ hipError_t run_refine(epseon_ctx* ctx, hipStream_t stream, hipStream_t stream_b,
                              ctx->waves_per_block, ctx->d_brackets, ctx->d_points, rel_tol, max_iter,
                              ctx->d_levels, ctx->d_status, ctx->d_iters, ctx->d_steps);
     }
-    const double* tab = lanes == 64 && ctx->segtab_ok ? (ctx->scan_windows ? ctx->d_segtab_band : ctx->d_segtab_full)
-                                                     : nullptr;
+    const double* tab = nullptr;
+    if (lanes == 64 && ctx->segtab_ok)
+        tab = ctx->scan_windows ? ctx->d_segtab_band : ctx->d_segtab_full;
+    else if (lanes == ctx->wide_lanes && ctx->scan_windows == ctx->wide_band)
+        tab = ctx->d_segtab_wide;
     const bool whole = ctx->xcd_scan && k0 == 0 && k1 == ctx->cum_level_tasks.size() - 1;
     const int32_t lpb = segmented_levels(ctx, lanes);
     ctx->last_refine_levels = lpb;

@@ -1598,36 +1598,49 @@ __device__ __forceinline__ void walk_tail(const double (&buf)[C], const int32_t 
 constexpr int32_t kBufferResourceWord3 = 0x00020000;
 
 // Grid values of one segment, value j being the j-th step's point (j
-// wave-uniform).  RowSource reads the natural uv table (lane-private
-// addresses); ColumnSource reads the lane's column of the segment table
-// through a wave-uniform buffer resource (row r at byte off + r * 512: the
-// lane's column offset in the vector offset, the row's in the scalar offset),
-// so each load instruction of a wavefront covers 512 contiguous bytes and
-// needs no address arithmetic on the vector ALU.
+// wave-uniform), loaded C at a time from an even j.  RowSource reads the
+// natural uv table (lane-private addresses); ColumnSource reads the lane's
+// column of the segment table, two steps per load, through a wave-uniform
+// buffer resource (row pair r at byte off + r * 16 T: the lane's column offset
+// in the vector offset, the pair's in the scalar offset), so each load
+// instruction of a wavefront covers 1024 contiguous bytes and needs no address
+// arithmetic on the vector ALU.
 struct RowSource {
     const double* p;
-    __device__ __forceinline__ double at(const int32_t j) const { return p[j]; }
+    template <int C>
+    __device__ __forceinline__ void load(double (&buf)[C], const int32_t j) const
+    {
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            buf[k] = p[j + k];
+    }
 };
 
+template <int T>
 struct ColumnSource {
     __amdgpu_buffer_rsrc_t rs;
     int32_t off;
-    __device__ __forceinline__ double row(const int32_t r) const
+    __device__ __forceinline__ double2 pair(const int32_t r) const
     {
-        typedef int32_t v2i __attribute__((ext_vector_type(2)));
-        const v2i x = __builtin_amdgcn_raw_buffer_load_b64(rs, off, r * 512, 0);
-        return __builtin_bit_cast(double, x);
+        typedef int32_t v4i __attribute__((ext_vector_type(4)));
+        const v4i x = __builtin_amdgcn_raw_buffer_load_b128(rs, off, r * (16 * T), 0);
+        return __builtin_bit_cast(double2, x);
     }
-    __device__ __forceinline__ double at(const int32_t j) const { return row(j + 1); }
-};
-
-template <int C, class Src>
-__device__ __forceinline__ void load_chunk(double (&buf)[C], const Src& src, const int32_t j)
-{
+    // The segment's first point.
+    __device__ __forceinline__ double first() const { return pair(0).y; }
+    template <int C>
+    __device__ __forceinline__ void load(double (&buf)[C], const int32_t j) const
+    {
+        static_assert(C % 2 == 0, "row pairs");
+        const int32_t r = (j >> 1) + 1;
 #pragma unroll
-    for (int k = 0; k < C; ++k)
-        buf[k] = src.at(j + k);
-}
+        for (int k = 0; k < C / 2; ++k) {
+            const double2 x = pair(r + k);
+            buf[2 * k] = x.x;
+            buf[2 * k + 1] = x.y;
+        }
+    }
+};
 
 // Visit the `len` values src.at(0 .. len - 1) in order, body(value, index);
 // ulen is wave-uniform with ulen <= len <= ulen + 1 (segment lengths differ by
@@ -1640,20 +1653,20 @@ template <int C, class Src, class Body>
 __device__ __forceinline__ void walk_segment(const Src& src, const int32_t len, const int32_t ulen, Body& body)
 {
     double A[C], B[C], D[C];
-    load_chunk(A, src, 0);
-    load_chunk(B, src, C);
+    src.load(A, 0);
+    src.load(B, C);
     int32_t j = 0;
     for (; j + 3 * C <= ulen; j += 3 * C) {
-        load_chunk(D, src, j + 2 * C);
+        src.load(D, j + 2 * C);
         walk_chunk(A, j, body);
-        load_chunk(A, src, j + 3 * C);
+        src.load(A, j + 3 * C);
         walk_chunk(B, j + C, body);
-        load_chunk(B, src, j + 4 * C);
+        src.load(B, j + 4 * C);
         walk_chunk(D, j + 2 * C, body);
     }
     const int32_t rem = ulen - j;
     if (rem >= 2 * C) {
-        load_chunk(D, src, j + 2 * C);
+        src.load(D, j + 2 * C);
         walk_chunk(A, j, body);
         walk_chunk(B, j + C, body);
         walk_tail(D, j + 2 * C, len, body);
@@ -1759,45 +1772,50 @@ struct CountBody {
 
 }  // namespace
 
-// Segment tables of the 64-lane segmented refinement: for job J, rows
-// r < seg_rows(J.n) of 64 columns from row J.seg_row, column s holding the
-// window's uv at point min(q0_s + r, n - 1) for the segments s < seg_count(n)
-// (zero in the unused columns).  One workgroup per 64-row tile of a job: each
+// Segment tables of the segmented refinement in `lanes`-lane blocks: for job
+// J, rows r < seg_rows(J.n) of `lanes` columns from row J.seg_row, column s
+// holding the window's uv at point min(q0_s + r - 1, n - 1) for the segments s
+// < seg_count(n) (zero in row 0 of the first and in the unused columns).  Rows
+// 2 p and 2 p + 1 are interleaved, so a lane reads two steps with one load.
+// One workgroup per tile of 64 rows and 64 columns (blockIdx.z) of a job: each
 // wavefront reads 64 consecutive points of one segment per load (512
 // contiguous bytes), the tile is transposed through LDS, and each wavefront
-// then stores 64 consecutive values of one row.
+// then stores 64 consecutive value pairs of two rows.
 constexpr int32_t kTableTile = 64;
 __global__ __launch_bounds__(256) void segment_table_kernel(const double* __restrict__ uv,
                                                             const PotentialRecord* __restrict__ pots,
                                                             const TableJob* __restrict__ jobs,
-                                                            const int32_t n_jobs, double* __restrict__ segtab)
+                                                            const int32_t n_jobs, const int32_t lanes,
+                                                            double* __restrict__ segtab)
 {
     __shared__ double tile[64][kTableTile + 1];
     const int32_t lane = static_cast<int32_t>(threadIdx.x & 63);
     const int32_t wave = static_cast<int32_t>(threadIdx.x >> 6);
+    const int32_t c0 = static_cast<int32_t>(blockIdx.z) * 64;
     for (int32_t jb = static_cast<int32_t>(blockIdx.y); jb < n_jobs; jb += static_cast<int32_t>(gridDim.y)) {
         const TableJob J = jobs[jb];
         const int32_t n = J.n;
-        const int32_t rows = seg_rows(n, 0, 1);
+        const int32_t rows = seg_rows(n, 0, 1, lanes);
         const int32_t qn = n - 2;
-        const int32_t segs = seg_count(n);
+        const int32_t segs = seg_count(n, lanes);
         const double* u = uv + pots[J.potential].ut_offset + J.lo;
-        double* out = segtab + static_cast<int64_t>(J.seg_row) * 64;
+        double2* out = reinterpret_cast<double2*>(segtab + static_cast<int64_t>(J.seg_row) * lanes) + c0;
         for (int32_t r0 = static_cast<int32_t>(blockIdx.x) * kTableTile; r0 < rows;
              r0 += static_cast<int32_t>(gridDim.x) * kTableTile) {
-            // Columns: wavefront w reads segments w, w + 4, ...; lane = row.
+            // Columns: wavefront w reads segments c0 + w, c0 + w + 4, ...; lane = row.
             for (int32_t sg = wave; sg < 64; sg += 4) {
                 double x = 0.0;
-                if (sg < segs) {
-                    const int64_t q = segment_start(qn, segs, sg) + r0 + lane;
-                    x = u[q < n - 1 ? q : n - 1];
+                if (c0 + sg < segs) {
+                    const int64_t q = segment_start(qn, segs, c0 + sg) + r0 + lane - 1;
+                    if (q >= 0)
+                        x = u[q < n - 1 ? q : n - 1];
                 }
                 tile[sg][lane] = x;
             }
             __syncthreads();
-            // Rows: wavefront w stores rows r0 + w, r0 + w + 4, ...; lane = column.
-            for (int32_t r = wave; r < kTableTile && r0 + r < rows; r += 4)
-                out[static_cast<int64_t>(r0 + r) * 64 + lane] = tile[lane][r];
+            // Row pairs: wavefront w stores pairs w, w + 4, ...; lane = column.
+            for (int32_t r = 2 * wave; r < kTableTile && r0 + r < rows; r += 8)
+                out[static_cast<int64_t>((r0 + r) >> 1) * lanes + lane] = make_double2(tile[lane][r], tile[lane][r + 1]);
             __syncthreads();
         }
     }
@@ -1820,18 +1838,18 @@ struct SegShared {
 // One level's shot geometry in a T-thread block: its band window (Dirichlet
 // points lo, hi on the trimmed grid), the q = n - 2 steps split into `segs`
 // segments, lane s walking [q0, q1) from the table value u_start.
-template <bool TABLE>
+template <int T, bool TABLE>
 struct SegGeom {
     const double* u;
     int32_t lo, hi, seg_row, n, qn, segs, q0, q1, ulen;
     bool active;
     double u_start;
-    ColumnSource cs;
+    ColumnSource<T> cs;
 
     // Lane `lane`'s steps [q0, q1) of the window (once per level):
     // floor(s q / sg) = s (q / sg) + floor(s (q mod sg) / sg), so 32-bit
     // arithmetic gives segment_start's values (s (q mod sg) < 2^16).
-    static __device__ __forceinline__ int2 bounds(const BandWindow& B, const int32_t lane, const int32_t T)
+    static __device__ __forceinline__ int2 bounds(const BandWindow& B, const int32_t lane)
     {
         const int32_t q = B.hi - B.lo - 1;
         const int32_t sg = min(T, max(1, q / 32));
@@ -1842,7 +1860,7 @@ struct SegGeom {
     }
 
     __device__ __forceinline__ void init(const double* uv_pot, const double* segtab, const BandWindow& B,
-                                         const int2 qb, const int32_t lane, const int32_t T)
+                                         const int2 qb, const int32_t lane)
     {
         lo = B.lo;
         hi = B.hi;
@@ -1856,22 +1874,23 @@ struct SegGeom {
         q1 = qb.y;
         // Every segment has qn / segs or qn / segs + 1 steps.
         ulen = __builtin_amdgcn_readfirstlane(qn / segs);
-        cs = ColumnSource{};
+        cs = ColumnSource<T>{};
         if constexpr (TABLE) {
-            // With the segment table, lane s reads column s (row r = point
-            // q0 + r): consecutive lanes load consecutive addresses.  The
+            // With the segment table, lane s reads column s: consecutive lanes
+            // load consecutive addresses.  The
             // resource must be wave-uniform (scalar registers); the
             // readfirstlane calls state what the compiler cannot prove.
-            const int32_t rows = seg_rows(n, 0, 1);
-            const uint64_t base = reinterpret_cast<uint64_t>(segtab + static_cast<int64_t>(B.seg_row) * 64);
+            const int32_t rows = seg_rows(n, 0, 1, T);
+            const int32_t row0 = T == 64 ? B.seg_row : B.wide_row;
+            const uint64_t base = reinterpret_cast<uint64_t>(segtab + static_cast<int64_t>(row0) * T);
             const uint32_t blo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
             const uint32_t bhi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32));
-            const int32_t bytes = __builtin_amdgcn_readfirstlane(rows * 512);
+            const int32_t bytes = __builtin_amdgcn_readfirstlane(rows * (8 * T));
             cs.rs = __builtin_amdgcn_make_buffer_rsrc(
                 reinterpret_cast<double*>((static_cast<uint64_t>(bhi) << 32) | blo), static_cast<int16_t>(0),
                 bytes, kBufferResourceWord3);
-            cs.off = lane * 8;
-            u_start = cs.row(0);
+            cs.off = lane * 16;
+            u_start = cs.first();
         } else {
             u_start = u[q0];
         }
@@ -2043,7 +2062,7 @@ __device__ __forceinline__ int32_t join_counts(const SegShared<T>& sh, const int
 // node count across segment borders.  In 64-lane blocks (one wavefront) the
 // tree runs in registers.
 template <int T, int KK, bool TABLE>
-__device__ __forceinline__ void segmented_shot(SegShared<T>& sh, const SegGeom<TABLE>& g, const int32_t lane,
+__device__ __forceinline__ void segmented_shot(SegShared<T>& sh, const SegGeom<T, TABLE>& g, const int32_t lane,
                                                const double (&e)[KK], const bool counted, const int32_t stride,
                                                const StepConsts& k, double (&fw)[KK], int32_t (&fk)[KK],
                                                int32_t& c)
@@ -2265,7 +2284,7 @@ numerov_refine_segmented_kernel(const double* __restrict__ uv, const double* __r
 #pragma unroll
     for (int q = 0; q < K; ++q) {
         band[q] = __builtin_amdgcn_readfirstlane(ctl.live[q] ? ctl.r[q].b.band : 0);
-        qb[q] = ctl.live[q] ? SegGeom<TABLE>::bounds(W[band[q]], lane, T) : make_int2(0, 0);
+        qb[q] = ctl.live[q] ? SegGeom<T, TABLE>::bounds(W[band[q]], lane) : make_int2(0, 0);
         wid[q] = q;
 #pragma unroll
         for (int o = q - 1; o >= 0; --o) {
@@ -2387,8 +2406,8 @@ numerov_refine_segmented_kernel(const double* __restrict__ uv, const double* __r
                     rest &= rest - 1;
                 }
             }
-            SegGeom<TABLE> g;
-            g.init(uv_pot, segtab, W[band0], qb0, lane, T);
+            SegGeom<T, TABLE> g;
+            g.init(uv_pot, segtab, W[band0], qb0, lane);
             int32_t c = 0;
             double fw[4];
             int32_t fk[4];
@@ -2562,7 +2581,8 @@ hipError_t launch_refine(hipStream_t stream, int32_t levels_per_lane, const doub
     return hipGetLastError();
 }
 
-// segtab != nullptr selects the segment tables for 64-lane blocks.
+// segtab: the segment tables for blocks of that many lanes, or null (segments
+// read from the natural table, lane by lane).
 // levels_per_block 2 or 4 (64-lane blocks only) takes tasks of that many
 // consecutive levels each.
 // bins == nullptr: tasks[0, n_tasks) in order; else `bins` (device, 9
@@ -2585,10 +2605,16 @@ hipError_t launch_refine_segmented(hipStream_t stream, int32_t lanes, int32_t le
                        levels, status, iterations, steps)
     switch (lanes) {
     case 256:
-        EPSEON_SEGMENTED(256, false, 1);
+        if (segtab != nullptr)
+            EPSEON_SEGMENTED(256, true, 1);
+        else
+            EPSEON_SEGMENTED(256, false, 1);
         break;
     case 128:
-        EPSEON_SEGMENTED(128, false, 1);
+        if (segtab != nullptr)
+            EPSEON_SEGMENTED(128, true, 1);
+        else
+            EPSEON_SEGMENTED(128, false, 1);
         break;
     case 64:
         if (levels_per_block == 4) {
@@ -2615,13 +2641,15 @@ hipError_t launch_refine_segmented(hipStream_t stream, int32_t lanes, int32_t le
 }
 
 hipError_t launch_segment_tables(hipStream_t stream, const double* uv, const PotentialRecord* pots,
-                                 const TableJob* jobs, int32_t n_jobs, int32_t max_rows, double* segtab)
+                                 const TableJob* jobs, int32_t n_jobs, int32_t max_rows, int32_t lanes,
+                                 double* segtab)
 {
     if (n_jobs == 0 || max_rows == 0)
         return hipSuccess;
     const int32_t bx = (max_rows + kTableTile - 1) / kTableTile;
-    dim3 grid(static_cast<unsigned>(bx < 1024 ? bx : 1024), static_cast<unsigned>(n_jobs < 65535 ? n_jobs : 65535));
-    hipLaunchKernelGGL(segment_table_kernel, grid, dim3(256), 0, stream, uv, pots, jobs, n_jobs, segtab);
+    dim3 grid(static_cast<unsigned>(bx < 1024 ? bx : 1024), static_cast<unsigned>(n_jobs < 65535 ? n_jobs : 65535),
+              static_cast<unsigned>(lanes / 64));
+    hipLaunchKernelGGL(segment_table_kernel, grid, dim3(256), 0, stream, uv, pots, jobs, n_jobs, lanes, segtab);
     return hipGetLastError();
 }
 

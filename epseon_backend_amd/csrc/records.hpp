@@ -92,26 +92,29 @@ struct ChunkEdge {
     int32_t first, last;
 };
 
-// Segments of the 64-lane segmented refinement of a potential with n points:
-// the q = n - 2 steps split into min(64, max(1, q / 32)) segments, segment s
-// covering steps [s q / segs, (s + 1) q / segs).
-constexpr int32_t seg_count(const int32_t n_points)
+// Segments of the segmented refinement of a window with n points in `lanes`
+// lanes: the q = n - 2 steps split into min(lanes, max(1, q / 32)) segments,
+// segment s covering steps [s q / segs, (s + 1) q / segs).
+constexpr int32_t seg_count(const int32_t n_points, const int32_t lanes)
 {
     const int32_t q = n_points - 2;
     const int32_t s = q / 32;
-    return s < 1 ? 1 : (s > 64 ? 64 : s);
+    return s < 1 ? 1 : (s > lanes ? lanes : s);
 }
 
-// Rows of a potential's segment table (row r of column s holds uv at point
-// q0_s + r): the longest segment plus the row of its start point and the 32
-// rows its walk reads ahead; none for a potential without levels to refine.
-constexpr int32_t seg_rows(const int32_t n_points, const int32_t flags, const int32_t level_count)
+// Rows of a window's segment table (row r of column s holds uv at point
+// q0_s + r - 1): a row of padding, so that a step's row pair starts at an even
+// row, the longest segment plus the row of its start point, and the 32 rows its
+// walk reads ahead, rounded up to whole pairs; none for a potential without
+// levels to refine.
+constexpr int32_t seg_rows(const int32_t n_points, const int32_t flags, const int32_t level_count,
+                           const int32_t lanes = 64)
 {
     if (flags != 0 || level_count <= 0)
         return 0;
     const int32_t q = n_points - 2;
-    const int32_t segs = seg_count(n_points);
-    return (q + segs - 1) / segs + 33;
+    const int32_t segs = seg_count(n_points, lanes);
+    return ((q + segs - 1) / segs + 35) & ~1;
 }
 
 // Segment length of the eigenfunction shots of a potential with n points: a
@@ -214,14 +217,16 @@ constexpr int kWindowDepth = 15;
 // One band window of a potential: Dirichlet points lo, hi (on the trimmed
 // grid) and the far-end scale of its n = hi - lo + 1 point scan shots
 // (12^(n-2) = far_scale 2^far_exp); seg_row is the first row of its segment
-// table.
+// table for 64-lane blocks, wide_row that of its table for the wider blocks
+// the batch refines in.
 struct BandWindow {
     int32_t lo, hi;
     int32_t far_exp;
     int32_t seg_row;
     double far_scale;
+    int32_t wide_row, pad;
 };
-static_assert(sizeof(BandWindow) == 24, "window layout");
+static_assert(sizeof(BandWindow) == 32, "window layout");
 
 // One segment table to build: the n-point window from point lo of a
 // potential's trimmed grid, stored from row seg_row.
