@@ -298,6 +298,34 @@ def _as_f64(a: np.ndarray) -> np.ndarray:
     return np.ascontiguousarray(a, dtype=np.float64)
 
 
+_DESC_DTYPE = np.dtype([("n_points", np.int64), ("n_energies", np.int64), ("r_min", np.float64),
+                        ("r_max", np.float64), ("reduced_mass", np.float64), ("e_top", np.float64),
+                        ("level_min", np.int32), ("level_count", np.int32)])
+
+
+def _descriptors(potentials: Sequence[Potential], points: Sequence[int]) -> np.ndarray:
+    """The batch's PotentialDesc records (at least one), filled column by column."""
+    n = len(potentials)
+    desc = np.zeros(max(n, 1), dtype=_DESC_DTYPE)
+    d = desc[:n]
+    d["n_points"] = points
+    d["n_energies"] = [int(p.n_energies) for p in potentials]
+    for name in ("r_min", "r_max", "reduced_mass", "e_top"):
+        d[name] = [float(getattr(p, name)) for p in potentials]
+    # Out-of-range level numbers wrap, as in the C struct.
+    for name in ("level_min", "level_count"):
+        d[name] = np.array([int(getattr(p, name)) for p in potentials], dtype=np.int64).astype(np.int32)
+    return desc
+
+
+def _offsets(points: Sequence[int]) -> np.ndarray:
+    """Start of each table in the concatenated batch (at least one entry)."""
+    offsets = np.zeros(max(len(points), 1), dtype=np.int64)
+    if len(points) > 1:
+        offsets[1:] = np.cumsum(points[:-1])
+    return offsets
+
+
 class Context:
     """One device context (stream + arena) of libepseon_hip."""
 
@@ -311,11 +339,13 @@ class Context:
         self.energy_counts: list[int] = []
         self.point_counts: list[int] = []
         self.v_offsets: list[int] = []
+        self._tables = np.empty(1, dtype=np.float64)
 
     def close(self) -> None:
         if self._h:
             self._lib.epseon_ctx_destroy(self._h)
             self._h = ctypes.c_void_p()
+            self._tables = np.empty(1, dtype=np.float64)
 
     def __enter__(self) -> Context:
         return self
@@ -331,66 +361,49 @@ class Context:
 
     def load(self, potentials: Sequence[Potential]) -> None:
         """Upload a batch (epseon_load_potentials)."""
-        n = len(potentials)
-        descs = (PotentialDesc * max(n, 1))()
-        offsets = np.zeros(max(n, 1), dtype=np.int64)
-        total = 0
-        for i, p in enumerate(potentials):
-            offsets[i] = total
-            total += len(p.values)
-        v = np.zeros(max(total, 1), dtype=np.float64)
-        for i, p in enumerate(potentials):
-            vals = _as_f64(p.values)
-            v[offsets[i] : offsets[i] + len(vals)] = vals
-            d = descs[i]
-            d.n_points = len(vals)
-            d.n_energies = int(p.n_energies)
-            d.r_min = float(p.r_min)
-            d.r_max = float(p.r_max)
-            d.reduced_mass = float(p.reduced_mass)
-            d.e_top = float(p.e_top)
-            d.level_min = int(p.level_min)
-            d.level_count = int(p.level_count)
+        values = [_as_f64(p.values) for p in potentials]
+        points = [len(v) for v in values]
+        offsets = _offsets(points)
+        # One table buffer per context, kept while it is large enough: a new
+        # one of this size costs more in page faults than the copy.
+        total = sum(points)
+        if len(self._tables) < total:
+            self._tables = np.empty(total, dtype=np.float64)
+        v = self._tables[: max(total, 1)]
+        if total > 0:
+            np.concatenate(values, out=v)
+        desc = _descriptors(potentials, points)
         _check(
             self._lib.epseon_load_potentials(
                 self._h,
-                n,
-                descs,
+                len(potentials),
+                desc.ctypes.data_as(ctypes.POINTER(PotentialDesc)),
                 v.ctypes.data_as(_c_double_p),
                 offsets.ctypes.data_as(_c_int64_p),
             )
         )
-        self.n_potentials = n
-        self.level_counts = [int(p.level_count) for p in potentials]
-        self.energy_counts = [int(p.n_energies) for p in potentials]
-        self.point_counts = [len(p.values) for p in potentials]
-        self.v_offsets = [int(o) for o in offsets[:n]]
+        self._loaded(desc, points, offsets)
 
     def load_device(self, potentials: Sequence[Potential], v_ptr: int, offsets: Sequence[int]) -> None:
         """Upload a batch whose V tables are already in device memory at
         v_ptr (doubles, potential p at offsets[p]; epseon_load_potentials_device).
         ``Potential.values`` may be any sized object: only its length is used."""
-        n = len(potentials)
-        descs = (PotentialDesc * max(n, 1))()
-        offs = np.zeros(max(n, 1), dtype=np.int64)
-        for i, p in enumerate(potentials):
-            offs[i] = int(offsets[i])
-            d = descs[i]
-            d.n_points = len(p.values)
-            d.n_energies = int(p.n_energies)
-            d.r_min = float(p.r_min)
-            d.r_max = float(p.r_max)
-            d.reduced_mass = float(p.reduced_mass)
-            d.e_top = float(p.e_top)
-            d.level_min = int(p.level_min)
-            d.level_count = int(p.level_count)
-        _check(self._lib.epseon_load_potentials_device(self._h, n, descs, ctypes.c_void_p(v_ptr),
-                                                       offs.ctypes.data_as(_c_int64_p)))
+        points = [len(p.values) for p in potentials]
+        offs = np.zeros(max(len(points), 1), dtype=np.int64)
+        offs[: len(points)] = [int(offsets[i]) for i in range(len(points))]
+        desc = _descriptors(potentials, points)
+        _check(self._lib.epseon_load_potentials_device(self._h, len(potentials),
+                                                       desc.ctypes.data_as(ctypes.POINTER(PotentialDesc)),
+                                                       ctypes.c_void_p(v_ptr), offs.ctypes.data_as(_c_int64_p)))
+        self._loaded(desc, points, offs)
+
+    def _loaded(self, desc: np.ndarray, points: list[int], offsets: np.ndarray) -> None:
+        n = len(points)
         self.n_potentials = n
-        self.level_counts = [int(p.level_count) for p in potentials]
-        self.energy_counts = [int(p.n_energies) for p in potentials]
-        self.point_counts = [len(p.values) for p in potentials]
-        self.v_offsets = [int(o) for o in offs[:n]]
+        self.level_counts = desc["level_count"][:n].tolist()
+        self.energy_counts = desc["n_energies"][:n].tolist()
+        self.point_counts = points
+        self.v_offsets = offsets[:n].tolist()
 
     def potential_info(self, p: int) -> PotentialInfo:
         info = PotentialInfo()

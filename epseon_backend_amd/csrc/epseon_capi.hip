@@ -44,6 +44,7 @@ hipError_t launch_refine_segmented(hipStream_t, int32_t, int32_t, const double*,
                                    double*, int32_t*, int32_t*, int32_t*);
 hipError_t launch_segment_tables(hipStream_t, const double*, const PotentialRecord*, const TableJob*,
                                  int32_t, int32_t, int32_t, double*);
+hipError_t launch_task_lists(hipStream_t, const TaskRun*, int32_t, WaveTask*, const PsiRun*, int32_t, PsiTask*);
 hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord*, int32_t, int64_t,
                                const ChunkEdge*, int2*);
 hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, int32_t, const int32_t*, const int32_t*,
@@ -177,6 +178,11 @@ constexpr int64_t kQuadMinLevelsPerCu = 96;
 // 160,000 184 and 140; 8 x 80 levels in 128 lanes, 20,000 points 60 and 54.
 // Below, the pass that builds them costs what they save.
 constexpr int32_t kWideTableMinPoints = 16384;
+
+// Host batches of this many points get their V statistics on the device: the
+// host walk takes 0.65 ns a point, the two passes and their read-back 50 us
+// and little more.
+constexpr int64_t kDeviceStatsMinPoints = 100000;
 
 // Automatic windows need at least this many scan wavefronts per SIMD.
 constexpr int64_t kWindowsMinScanWavesPerSimd = 8;
@@ -403,6 +409,8 @@ struct epseon_ctx {
     size_t stage_elems = 0;
     int64_t user_span = 0;
     int64_t psi_total = 0;
+    // A load's host arrays on their way to the device (kept for the next load).
+    std::vector<char> h_upload;
     // Position of each potential in task order.
     std::vector<int32_t> order_pos;
 
@@ -630,80 +638,106 @@ hipError_t build_tables(epseon_ctx* ctx, hipStream_t stream, bool band)
 // Shared body of epseon_load_potentials (v_host) and
 // epseon_load_potentials_device (v_dev).
 // Band of the scan group starting at trial energy j0 (as the kernels
-// compute it).
-int32_t host_group_band(const PotentialRecord& r, int32_t j0)
+// compute it), at or above `from` (the band of an earlier group, or 0).
+int32_t host_group_band(const PotentialRecord& r, int32_t j0, int32_t from)
 {
     const int32_t jt = std::min(j0 + 63, r.n_energies - 1);
     const double et = std::fma(static_cast<double>(jt + 1), r.de, r.e_lo);
     const double step = (r.e_hi - r.e_lo) / kBands;
-    for (int32_t b = 0; b < kBands - 1; ++b)
+    for (int32_t b = from; b < kBands - 1; ++b)
         if (std::fma(static_cast<double>(b + 1), step, r.e_lo) >= et)
             return b;
     return kBands - 1;
 }
 
-// Per-XCD bins of a task list (potentials in task order, potential k's
-// tasks at [cum[k], cum[k + 1]), task t worth work[t]).  Each potential's
-// tasks are cut into chunks of at most ceil(tasks / 32) (so a single large
-// potential still spreads over every XCD, while typical batch members stay
-// whole); chunks go by decreasing work to the least-loaded bin.  Each bin
-// keeps the chunks in task order (a potential's tasks stay together, so its
-// table stays in that XCD's L2); with `longest_first` the tasks of each
-// chunk go by decreasing work (stable).  Returns the concatenated bins;
-// `bins` gets the 9 offsets and `max_bin` the largest bin's size.
-std::vector<WaveTask> xcd_binned(const std::vector<WaveTask>& tasks, const std::vector<int32_t>& cum,
-                                 const std::vector<double>& work, bool longest_first, std::vector<int32_t>& bins,
-                                 int32_t& max_bin)
+// Tasks [i0, i1) of the potential at task-order position k.
+struct TaskChunk {
+    int32_t k, i0, i1;
+};
+
+// Per-XCD bins of a task list (potentials in task order, cum[k] tasks before
+// potential k's; work(k, i0, i1) is the work of its tasks [i0, i1)).  Each
+// potential's tasks are cut into chunks of at most ceil(tasks / 32) (so a
+// single large potential still spreads over every XCD, while typical batch
+// members stay whole); chunks go by decreasing work to the least-loaded bin.
+// Each bin keeps the chunks in task order (a potential's tasks stay together,
+// so its table stays in that XCD's L2).  Returns the bins' chunks one bin
+// after the other; `bins` gets the 9 task offsets and `max_bin` the largest
+// bin's size.
+template <class Work>
+std::vector<TaskChunk> xcd_chunks(const std::vector<int32_t>& cum, const Work& work, std::vector<int32_t>& bins,
+                                  int32_t& max_bin)
 {
-    struct Chunk {
-        int32_t t0, t1;
-        double work;
-    };
-    std::vector<Chunk> chunks;
-    const int32_t cmax = std::max<int32_t>(1, (static_cast<int32_t>(tasks.size()) + 31) / 32);
+    std::vector<TaskChunk> chunks;
+    std::vector<double> load_of;
+    const int32_t cmax = std::max<int32_t>(1, (cum.back() + 31) / 32);
     for (size_t k = 0; k + 1 < cum.size(); ++k)
-        for (int32_t t = cum[k]; t < cum[k + 1]; t += cmax) {
-            const int32_t e = std::min(cum[k + 1], t + cmax);
-            double w = 0.0;
-            for (int32_t i = t; i < e; ++i)
-                w += work[static_cast<size_t>(i)];
-            chunks.push_back({t, e, w});
+        for (int32_t i = 0, n = cum[k + 1] - cum[k]; i < n; i += cmax) {
+            chunks.push_back({static_cast<int32_t>(k), i, std::min(n, i + cmax)});
+            load_of.push_back(work(k, chunks.back().i0, chunks.back().i1));
         }
-    std::vector<size_t> by_work(chunks.size());
-    std::iota(by_work.begin(), by_work.end(), size_t(0));
-    std::stable_sort(by_work.begin(), by_work.end(),
-                     [&](size_t a, size_t b) { return chunks[a].work > chunks[b].work; });
-    std::vector<int32_t> chunk_bin(chunks.size(), 0);
+    std::vector<int32_t> by_work(chunks.size());
+    std::iota(by_work.begin(), by_work.end(), 0);
+    std::stable_sort(by_work.begin(), by_work.end(), [&](int32_t a, int32_t b) {
+        return load_of[static_cast<size_t>(a)] > load_of[static_cast<size_t>(b)];
+    });
+    std::vector<uint8_t> bin_of(chunks.size());
     double load[8] = {};
-    for (size_t c : by_work) {
-        const int x = static_cast<int>(std::min_element(load, load + 8) - load);
-        chunk_bin[c] = x;
-        load[x] += chunks[c].work;
+    for (int32_t c : by_work) {
+        const size_t x = static_cast<size_t>(std::min_element(load, load + 8) - load);
+        bin_of[static_cast<size_t>(c)] = static_cast<uint8_t>(x);
+        load[x] += load_of[static_cast<size_t>(c)];
     }
-    std::vector<WaveTask> out;
-    out.reserve(tasks.size());
+    std::vector<TaskChunk> out;
+    out.reserve(chunks.size());
     bins.assign(9, 0);
     max_bin = 0;
-    for (int x = 0; x < 8; ++x) {
-        bins[static_cast<size_t>(x)] = static_cast<int32_t>(out.size());
-        for (size_t c = 0; c < chunks.size(); ++c) {  // chunks are in task order
-            if (chunk_bin[c] != x)
-                continue;
-            std::vector<int32_t> ids;
-            for (int32_t t = chunks[c].t0; t < chunks[c].t1; ++t)
-                ids.push_back(t);
-            if (longest_first)
-                std::stable_sort(ids.begin(), ids.end(), [&](int32_t a, int32_t b) {
-                    return work[static_cast<size_t>(a)] > work[static_cast<size_t>(b)];
-                });
-            for (int32_t t : ids)
-                out.push_back(tasks[static_cast<size_t>(t)]);
-        }
-        max_bin = std::max(max_bin, static_cast<int32_t>(out.size()) - bins[static_cast<size_t>(x)]);
+    int32_t tasks = 0;
+    for (size_t x = 0; x < 8; ++x) {
+        bins[x] = tasks;
+        for (size_t c = 0; c < chunks.size(); ++c)  // chunks are in task order
+            if (bin_of[c] == x) {
+                out.push_back(chunks[c]);
+                tasks += chunks[c].i1 - chunks[c].i0;
+            }
+        max_bin = std::max(max_bin, tasks - bins[x]);
     }
-    bins[8] = static_cast<int32_t>(out.size());
+    bins[8] = tasks;
     return out;
 }
+
+// Host arrays gathered into one buffer and sent to one device block: each
+// array starts at a multiple of 256 bytes (at least one element's room).
+class Packed {
+  public:
+    explicit Packed(std::vector<char>& buffer) : buf_(buffer) { buf_.clear(); }
+
+    template <typename T>
+    void add(const std::vector<T>& v, T** dev)
+    {
+        const size_t at = (buf_.size() + 255) & ~size_t(255);
+        const size_t bytes = v.size() * sizeof(T);
+        buf_.resize(at + std::max(bytes, sizeof(T)));
+        if (bytes > 0)
+            std::memcpy(buf_.data() + at, v.data(), bytes);
+        fix_.push_back({at, reinterpret_cast<void**>(dev)});
+    }
+
+    hipError_t send(Arena& a, hipStream_t stream)
+    {
+        char* base = nullptr;
+        if (const hipError_t e = arena_array(a, std::max<size_t>(buf_.size(), 1), &base); e != hipSuccess)
+            return e;
+        for (const auto& f : fix_)
+            *f.second = base + f.first;
+        return buf_.empty() ? hipSuccess
+                            : hipMemcpyAsync(base, buf_.data(), buf_.size(), hipMemcpyHostToDevice, stream);
+    }
+
+  private:
+    std::vector<char>& buf_;
+    std::vector<std::pair<size_t, void**>> fix_;
+};
 
 int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc, const double* v_host,
                const double* v_dev, const int64_t* v_offsets)
@@ -783,12 +817,24 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         max_table_chunks = std::max(max_table_chunks, tc);
     }
 
+    // V in the caller's layout: one upload of the whole span from the host,
+    // or the caller's device buffer itself (read only during this call).
+    const double* v_src = v_dev;
+    if (v_host != nullptr) {
+        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(user_span, 1)), &ctx->d_v));
+        v_src = ctx->d_v;
+        if (user_span > 0)
+            EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_v, v_host, static_cast<size_t>(user_span) * sizeof(double),
+                                          hipMemcpyHostToDevice, ctx->stream));
+    }
+
     // V statistics: min V, its first index, the wall-trimmed Dirichlet points
     // (the last point left of the minimum and the first point right of it
     // where V >= V_min + 1/(2 beta); inside, 1 + beta (E - V_i) > 1/2 for
-    // every E >= V_min) and the first non-finite value.
+    // every E >= V_min) and the first non-finite value.  Small host batches
+    // are walked here.
     std::vector<PotentialStats> vstats(static_cast<size_t>(std::max(count, 1)));
-    if (v_host != nullptr) {
+    if (v_host != nullptr && all_points < kDeviceStatsMinPoints) {
         for (int32_t p = 0; p < count; ++p) {
             const int64_t n = desc[p].n_points;
             const double* vp = v_host + v_offsets[p];
@@ -827,21 +873,15 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         PotentialStats* d_st = nullptr;
         int32_t* d_chunk0 = nullptr;
         ChunkMin* d_chunks = nullptr;
-        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_off));
-        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_cnt));
-        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_beta));
+        Packed up(ctx->h_upload);
+        up.add(std::vector<int64_t>(v_offsets, v_offsets + count), &d_off);
+        up.add(counts, &d_cnt);
+        up.add(betas, &d_beta);
+        up.add(stats_chunk0, &d_chunk0);
+        EPSEON_HIP_TRY(up.send(a, ctx->stream));
         EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_st));
-        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(count), &d_chunk0));
         EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(stats_chunks), &d_chunks));
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_off, v_offsets, count * sizeof(int64_t), hipMemcpyHostToDevice,
-                                      ctx->stream));
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_cnt, counts.data(), count * sizeof(int64_t),
-                                      hipMemcpyHostToDevice, ctx->stream));
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_beta, betas.data(), count * sizeof(double),
-                                      hipMemcpyHostToDevice, ctx->stream));
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_chunk0, stats_chunk0.data(), count * sizeof(int32_t), hipMemcpyHostToDevice,
-                                      ctx->stream));
-        EPSEON_HIP_TRY(launch_potential_stats(ctx->stream, v_dev, d_off, d_cnt, d_chunk0, d_beta, count,
+        EPSEON_HIP_TRY(launch_potential_stats(ctx->stream, v_src, d_off, d_cnt, d_chunk0, d_beta, count,
                                               max_stats_chunks, d_chunks, d_st));
         EPSEON_HIP_TRY(hipMemcpyAsync(vstats.data(), d_st, count * sizeof(PotentialStats),
                                       hipMemcpyDeviceToHost, ctx->stream));
@@ -957,106 +997,125 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     ctx->order_pos.assign(static_cast<size_t>(count), 0);
     for (int32_t k = 0; k < count; ++k)
         ctx->order_pos[static_cast<size_t>(order[static_cast<size_t>(k)])] = k;
-    // Segmented refinement uses one 64-lane block per level.
-    std::vector<WaveTask> scan_tasks, refine_tasks, level_tasks, lane1_tasks, lane2_tasks, group_tasks[2];
-    std::vector<PsiTask> vjp_lists[4], psi_tasks;
-    ctx->cum_psi_tasks.assign(1, 0);
-    ctx->cum_lane1_tasks.assign(1, 0);
-    ctx->cum_lane2_tasks.assign(1, 0);
-    ctx->cum_scan_tasks.assign(1, 0);
-    ctx->cum_refine_tasks.assign(1, 0);
-    ctx->cum_level_tasks.assign(1, 0);
-    ctx->cum_group_tasks[0].assign(1, 0);
-    ctx->cum_group_tasks[1].assign(1, 0);
+    // The lists themselves are written on the device from runs of consecutive
+    // tasks, one run per potential and list or per chunk of a binned list.
+    std::vector<TaskRun> runs;
+    std::vector<PsiRun> psi_runs;
+    int64_t n_wave_tasks = 0, n_psi_tasks = 0;
+    const auto add_run = [&](int32_t p, int32_t first, int32_t step, int32_t n) {
+        if (n > 0)
+            runs.push_back({n_wave_tasks, p, first, step, n});
+        n_wave_tasks += n;
+    };
+    // One list: `tasks(r)` tasks of `step` energies or levels per potential.
+    const auto add_list = [&](std::vector<int32_t>& cum, int32_t step, const auto& tasks) {
+        cum.assign(1, 0);
+        const int64_t base = n_wave_tasks;
+        for (int32_t p : order) {
+            const int32_t n = tasks(ctx->rec[static_cast<size_t>(p)]);
+            add_run(p, 0, step, n);
+            cum.push_back(cum.back() + n);
+        }
+        return base;
+    };
+    const auto ceil_div = [](int32_t x, int32_t y) { return (x + y - 1) / y; };
+    const auto usable = [](const PotentialRecord& r) { return r.flags == EPSEON_POT_OK; };
+    const int64_t scan_at = add_list(ctx->cum_scan_tasks, 64, [&](const PotentialRecord& r) {
+        return usable(r) ? ceil_div(r.n_energies, 64) : 0;
+    });
+    const int64_t refine_at = add_list(ctx->cum_refine_tasks, 64,
+                                       [&](const PotentialRecord& r) { return ceil_div(r.level_count, 64); });
+    // Segmented refinement uses one block per level, or per group of levels.
+    const int64_t level_at =
+        add_list(ctx->cum_level_tasks, 1, [](const PotentialRecord& r) { return r.level_count; });
+    const int64_t lane1_at = add_list(ctx->cum_lane1_tasks, 64, [](const PotentialRecord& r) {
+        return r.level_count > 0 && r.level_count <= 64 ? 1 : 0;
+    });
+    const int64_t lane2_at = add_list(ctx->cum_lane2_tasks, 128, [&](const PotentialRecord& r) {
+        return r.level_count > 64 ? ceil_div(r.level_count, 128) : 0;
+    });
+    int64_t group_at[2];
+    for (int32_t g = 0; g < 2; ++g)
+        group_at[g] = add_list(ctx->cum_group_tasks[g], 2 << g,
+                               [&](const PotentialRecord& r) { return ceil_div(r.level_count, 2 << g); });
     ctx->cum_scan_work.assign(1, 0.0);
     for (int32_t p : order) {
-        const int32_t groups = (ctx->rec[p].level_count + 63) / 64;
-        const PotentialRecord& r = ctx->rec[p];
-        {
-            // Unresolved potentials get one task (side 0, segment 0), which
-            // zeroes their rows and gradient.
-            std::vector<PsiTask>& vl = vjp_lists[std::clamp(groups, 1, 4) - 1];
-            const bool ok = r.flags == EPSEON_POT_OK;
-            for (int32_t side = 0; side < (ok ? 2 : 1); ++side) {
-                const int32_t segs = !ok ? 1 : (side == 0 ? r.psi_segs_left : r.psi_segs_right);
-                for (int32_t sg = 0; sg < segs; ++sg) {
-                    vl.push_back({p, 0, side, sg});
-                    for (int32_t l = 0; l < r.level_count; l += 64)
-                        psi_tasks.push_back({p, l, side, sg});
-                }
-            }
-            ctx->cum_psi_tasks.push_back(static_cast<int32_t>(psi_tasks.size()));
-        }
-        if (r.flags == EPSEON_POT_OK)
-            for (int32_t j = 0; j < r.n_energies; j += 64)
-                scan_tasks.push_back({p, j});
-        for (int32_t l = 0; l < r.level_count; l += 64)
-            refine_tasks.push_back({p, l});
-        for (int32_t l = 0; l < r.level_count; ++l)
-            level_tasks.push_back({p, l});
-        for (int32_t g = 0; g < 2; ++g)
-            for (int32_t l = 0; l < r.level_count; l += 2 << g)
-                group_tasks[g].push_back({p, l});
-        if (r.level_count > 64)
-            for (int32_t l = 0; l < r.level_count; l += 128)
-                lane2_tasks.push_back({p, l});
-        else if (r.level_count > 0)
-            lane1_tasks.push_back({p, 0});
-        ctx->cum_lane1_tasks.push_back(static_cast<int32_t>(lane1_tasks.size()));
-        ctx->cum_lane2_tasks.push_back(static_cast<int32_t>(lane2_tasks.size()));
-        ctx->cum_scan_tasks.push_back(static_cast<int32_t>(scan_tasks.size()));
-        ctx->cum_refine_tasks.push_back(static_cast<int32_t>(refine_tasks.size()));
-        ctx->cum_level_tasks.push_back(static_cast<int32_t>(level_tasks.size()));
-        for (int32_t g = 0; g < 2; ++g)
-            ctx->cum_group_tasks[g].push_back(static_cast<int32_t>(group_tasks[g].size()));
-        ctx->cum_scan_work.push_back(
-            ctx->cum_scan_work.back() +
-            (r.flags == EPSEON_POT_OK ? static_cast<double>(r.n_points) * r.n_energies : 0.0));
+        const PotentialRecord& r = ctx->rec[static_cast<size_t>(p)];
+        ctx->cum_scan_work.push_back(ctx->cum_scan_work.back() +
+                                     (usable(r) ? static_cast<double>(r.n_points) * r.n_energies : 0.0));
     }
-    ctx->n_scan_tasks = static_cast<int32_t>(scan_tasks.size());
-    // Work per task: trial energies times recurrence steps (whole grid) for
-    // the scan, grid points for a level's refinement.
-    std::vector<double> scan_task_work(scan_tasks.size()), level_task_work(level_tasks.size());
-    for (size_t t = 0; t < scan_tasks.size(); ++t) {
-        const PotentialRecord& r = ctx->rec[static_cast<size_t>(scan_tasks[t].potential)];
-        scan_task_work[t] = static_cast<double>(std::min(64, r.n_energies - scan_tasks[t].first)) *
-                            static_cast<double>(r.n_points - 2);
-    }
-    for (size_t t = 0; t < level_tasks.size(); ++t)
-        level_task_work[t] = static_cast<double>(ctx->rec[static_cast<size_t>(level_tasks[t].potential)].n_points);
-    std::vector<double> group_task_work[2];
-    for (int32_t g = 0; g < 2; ++g) {
-        group_task_work[g].resize(group_tasks[g].size());
-        for (size_t t = 0; t < group_tasks[g].size(); ++t) {
-            const PotentialRecord& r = ctx->rec[static_cast<size_t>(group_tasks[g][t].potential)];
-            group_task_work[g][t] =
-                static_cast<double>(r.n_points) * std::min(2 << g, r.level_count - group_tasks[g][t].first);
-        }
-    }
+    ctx->n_scan_tasks = ctx->cum_scan_tasks.back();
+    ctx->n_refine_tasks = ctx->cum_refine_tasks.back();
+    ctx->n_level_tasks = ctx->cum_level_tasks.back();
+    for (int32_t g = 0; g < 2; ++g)
+        ctx->n_group_tasks[g] = ctx->cum_group_tasks[g].back();
+
+    // The same lists binned per XCD: work is trial energies times recurrence
+    // steps (whole grid) for the scan, levels times grid points for the
+    // refinement.
+    const auto rec_at = [&](size_t k) -> const PotentialRecord& {
+        return ctx->rec[static_cast<size_t>(order[k])];
+    };
     std::vector<int32_t> xcd_bins, xcd_level_bins, xcd_group_bins[2];
-    const std::vector<WaveTask> xcd_tasks =
-        xcd_binned(scan_tasks, ctx->cum_scan_tasks, scan_task_work, false, xcd_bins, ctx->xcd_max_bin);
-    const std::vector<WaveTask> xcd_level_tasks = xcd_binned(level_tasks, ctx->cum_level_tasks, level_task_work,
-                                                             false, xcd_level_bins, ctx->xcd_max_level_bin);
-    std::vector<WaveTask> xcd_group_tasks[2];
+    const auto add_binned = [&](const std::vector<int32_t>& cum, int32_t step, const auto& work,
+                                std::vector<int32_t>& bins, int32_t& max_bin) {
+        const int64_t base = n_wave_tasks;
+        for (const TaskChunk& c : xcd_chunks(cum, work, bins, max_bin))
+            add_run(order[static_cast<size_t>(c.k)], c.i0 * step, step, c.i1 - c.i0);
+        return base;
+    };
+    const int64_t xcd_scan_at = add_binned(
+        ctx->cum_scan_tasks, 64,
+        [&](size_t k, int32_t i0, int32_t i1) {
+            const PotentialRecord& r = rec_at(k);
+            return static_cast<double>(std::min(64 * i1, r.n_energies) - 64 * i0) *
+                   static_cast<double>(r.n_points - 2);
+        },
+        xcd_bins, ctx->xcd_max_bin);
+    const auto level_work = [&](int32_t step) {
+        return [&rec_at, step](size_t k, int32_t i0, int32_t i1) {
+            const PotentialRecord& r = rec_at(k);
+            return static_cast<double>(r.n_points) * (std::min(step * i1, r.level_count) - step * i0);
+        };
+    };
+    const int64_t xcd_level_at =
+        add_binned(ctx->cum_level_tasks, 1, level_work(1), xcd_level_bins, ctx->xcd_max_level_bin);
+    int64_t xcd_group_at[2];
     for (int32_t g = 0; g < 2; ++g)
-        xcd_group_tasks[g] = xcd_binned(group_tasks[g], ctx->cum_group_tasks[g], group_task_work[g], false,
-                                        xcd_group_bins[g], ctx->xcd_max_group_bin[g]);
-    ctx->n_refine_tasks = static_cast<int32_t>(refine_tasks.size());
-    ctx->n_level_tasks = static_cast<int32_t>(level_tasks.size());
-    for (int32_t g = 0; g < 2; ++g)
-        ctx->n_group_tasks[g] = static_cast<int32_t>(group_tasks[g].size());
+        xcd_group_at[g] = add_binned(ctx->cum_group_tasks[g], 2 << g, level_work(2 << g), xcd_group_bins[g],
+                                     ctx->xcd_max_group_bin[g]);
+
+    // Adjoint tasks (potential, side, segment) by block width, then the
+    // eigenfunction tasks (potential, 64 levels, side, segment).  Unresolved
+    // potentials get one segment (side 0, segment 0), which zeroes their rows
+    // and gradient.
+    const auto add_psi = [&](int32_t p, int32_t groups) {
+        const PotentialRecord& r = ctx->rec[static_cast<size_t>(p)];
+        for (int32_t side = 0; side < (usable(r) ? 2 : 1); ++side) {
+            const int32_t segs = !usable(r) ? 1 : (side == 0 ? r.psi_segs_left : r.psi_segs_right);
+            if (segs * groups > 0)
+                psi_runs.push_back({n_psi_tasks, p, side, segs, groups});
+            n_psi_tasks += static_cast<int64_t>(segs) * groups;
+        }
+    };
+    int64_t vjp_at[4];
+    for (int32_t w = 0; w < 4; ++w) {
+        vjp_at[w] = n_psi_tasks;
+        for (int32_t p : order)
+            if (std::clamp((ctx->rec[static_cast<size_t>(p)].level_count + 63) / 64, 1, 4) == w + 1)
+                add_psi(p, 1);
+        ctx->n_vjp[w] = static_cast<int32_t>(n_psi_tasks - vjp_at[w]);
+    }
+    const int64_t psi_at = n_psi_tasks;
+    ctx->cum_psi_tasks.assign(1, 0);
+    for (int32_t p : order) {
+        add_psi(p, (ctx->rec[static_cast<size_t>(p)].level_count + 63) / 64);
+        ctx->cum_psi_tasks.push_back(static_cast<int32_t>(n_psi_tasks - psi_at));
+    }
 
     const size_t np = static_cast<size_t>(std::max<int64_t>(pts, 1));
     const size_t ne = static_cast<size_t>(std::max<int64_t>(en, 1));
     const size_t nl = static_cast<size_t>(std::max<int64_t>(lv, 1));
-    // V in the caller's layout: one upload of the whole span from the host,
-    // or the caller's device buffer itself (read only during this call).
-    const double* v_src = v_dev;
-    if (v_host != nullptr) {
-        EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(user_span, 1)), &ctx->d_v));
-        v_src = ctx->d_v;
-    }
     EPSEON_HIP_TRY(arena_array(a, np, &ctx->d_ut));
     EPSEON_HIP_TRY(arena_array(a, np, &ctx->d_uv));
     EPSEON_HIP_TRY(arena_array(a, np, &ctx->d_uvr));
@@ -1066,28 +1125,21 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     EPSEON_HIP_TRY(arena_array(a, nw, &d_raw_windows));
     ChunkEdge* d_edges = nullptr;
     EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max(table_chunks, 1)) * kBands, &d_edges));
-    EPSEON_HIP_TRY(arena_array(a, nw, &ctx->d_win_full));
-    EPSEON_HIP_TRY(arena_array(a, nw, &ctx->d_win_band));
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_brackets));
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_points));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(count, 1), &ctx->d_rec));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(scan_tasks.size(), 1), &ctx->d_scan_tasks));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(xcd_tasks.size(), 1), &ctx->d_xcd_scan_tasks));
-    EPSEON_HIP_TRY(arena_array(a, size_t(9), &ctx->d_xcd_bins));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(xcd_level_tasks.size(), 1), &ctx->d_xcd_level_tasks));
-    EPSEON_HIP_TRY(arena_array(a, size_t(9), &ctx->d_xcd_level_bins));
-    for (int32_t g = 0; g < 2; ++g) {
-        EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(group_tasks[g].size(), 1), &ctx->d_group_tasks[g]));
-        EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(xcd_group_tasks[g].size(), 1), &ctx->d_xcd_group_tasks[g]));
-        EPSEON_HIP_TRY(arena_array(a, size_t(9), &ctx->d_xcd_group_bins[g]));
+    WaveTask* d_wave_tasks = nullptr;
+    PsiTask* d_all_psi_tasks = nullptr;
+    EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(n_wave_tasks, 1)), &d_wave_tasks));
+    EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(n_psi_tasks, 1)), &d_all_psi_tasks));
+    {
+        // Scan results in one block, cleared together: far ends (f64), node
+        // and rescale counts (i32).
+        char* block = nullptr;
+        EPSEON_HIP_TRY(arena_array(a, ne * (sizeof(double) + 2 * sizeof(int32_t)), &block));
+        ctx->d_far = reinterpret_cast<double*>(block);
+        ctx->d_nodes = reinterpret_cast<int32_t*>(block + ne * sizeof(double));
+        ctx->d_resc = ctx->d_nodes + ne;
     }
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(refine_tasks.size(), 1), &ctx->d_refine_tasks));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(level_tasks.size(), 1), &ctx->d_level_tasks));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(lane1_tasks.size(), 1), &ctx->d_lane1_tasks));
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(lane2_tasks.size(), 1), &ctx->d_lane2_tasks));
-    EPSEON_HIP_TRY(arena_array(a, ne, &ctx->d_nodes));
-    EPSEON_HIP_TRY(arena_array(a, ne, &ctx->d_far));
-    EPSEON_HIP_TRY(arena_array(a, ne, &ctx->d_resc));
     {
         // One block: levels (f64), status, iterations (i32) and the summary
         // (3 i64), each 256-byte aligned, read back whole; then the steps
@@ -1104,73 +1156,36 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     }
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_norms));
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_grad_levels));
-    for (int w = 0; w < 4; ++w) {
-        ctx->n_vjp[w] = static_cast<int32_t>(vjp_lists[w].size());
-        EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(vjp_lists[w].size(), 1), &ctx->d_vjp_lists[w]));
-        if (!vjp_lists[w].empty())
-            EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_vjp_lists[w], vjp_lists[w].data(),
-                                          vjp_lists[w].size() * sizeof(PsiTask),
-                                          hipMemcpyHostToDevice, ctx->stream));
+    {
+        TaskRun* d_runs = nullptr;
+        PsiRun* d_psi_runs = nullptr;
+        Packed up(ctx->h_upload);
+        up.add(ctx->rec, &ctx->d_rec);
+        up.add(runs, &d_runs);
+        up.add(psi_runs, &d_psi_runs);
+        up.add(xcd_bins, &ctx->d_xcd_bins);
+        up.add(xcd_level_bins, &ctx->d_xcd_level_bins);
+        for (int32_t g = 0; g < 2; ++g)
+            up.add(xcd_group_bins[g], &ctx->d_xcd_group_bins[g]);
+        EPSEON_HIP_TRY(up.send(a, ctx->stream));
+        EPSEON_HIP_TRY(launch_task_lists(ctx->stream, d_runs, static_cast<int32_t>(runs.size()), d_wave_tasks,
+                                         d_psi_runs, static_cast<int32_t>(psi_runs.size()), d_all_psi_tasks));
     }
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(psi_tasks.size(), 1), &ctx->d_psi_tasks));
-    if (!psi_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_psi_tasks, psi_tasks.data(), psi_tasks.size() * sizeof(PsiTask),
-                                      hipMemcpyHostToDevice, ctx->stream));
-
-    if (v_host != nullptr && user_span > 0)
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_v, v_host, static_cast<size_t>(user_span) * sizeof(double),
-                                      hipMemcpyHostToDevice, ctx->stream));
-    if (count > 0)
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_rec, ctx->rec.data(),
-                                      static_cast<size_t>(count) * sizeof(PotentialRecord),
-                                      hipMemcpyHostToDevice, ctx->stream));
-    if (!scan_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_scan_tasks, scan_tasks.data(),
-                                      scan_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                      ctx->stream));
-    if (!xcd_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_scan_tasks, xcd_tasks.data(),
-                                      xcd_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                      ctx->stream));
-    if (!xcd_level_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_level_tasks, xcd_level_tasks.data(),
-                                      xcd_level_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                      ctx->stream));
-    EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_level_bins, xcd_level_bins.data(), 9 * sizeof(int32_t),
-                                  hipMemcpyHostToDevice, ctx->stream));
+    ctx->d_scan_tasks = d_wave_tasks + scan_at;
+    ctx->d_refine_tasks = d_wave_tasks + refine_at;
+    ctx->d_level_tasks = d_wave_tasks + level_at;
+    ctx->d_lane1_tasks = d_wave_tasks + lane1_at;
+    ctx->d_lane2_tasks = d_wave_tasks + lane2_at;
+    ctx->d_xcd_scan_tasks = d_wave_tasks + xcd_scan_at;
+    ctx->d_xcd_level_tasks = d_wave_tasks + xcd_level_at;
     for (int32_t g = 0; g < 2; ++g) {
-        if (!group_tasks[g].empty())
-            EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_group_tasks[g], group_tasks[g].data(),
-                                          group_tasks[g].size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                          ctx->stream));
-        if (!xcd_group_tasks[g].empty())
-            EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_group_tasks[g], xcd_group_tasks[g].data(),
-                                          xcd_group_tasks[g].size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                          ctx->stream));
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_group_bins[g], xcd_group_bins[g].data(), 9 * sizeof(int32_t),
-                                      hipMemcpyHostToDevice, ctx->stream));
+        ctx->d_group_tasks[g] = d_wave_tasks + group_at[g];
+        ctx->d_xcd_group_tasks[g] = d_wave_tasks + xcd_group_at[g];
     }
-    EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_bins, xcd_bins.data(), 9 * sizeof(int32_t),
-                                  hipMemcpyHostToDevice, ctx->stream));
-    if (!refine_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_refine_tasks, refine_tasks.data(),
-                                      refine_tasks.size() * sizeof(WaveTask),
-                                      hipMemcpyHostToDevice, ctx->stream));
-    if (!level_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_level_tasks, level_tasks.data(),
-                                      level_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                      ctx->stream));
-    if (!lane1_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_lane1_tasks, lane1_tasks.data(),
-                                      lane1_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                      ctx->stream));
-    if (!lane2_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_lane2_tasks, lane2_tasks.data(),
-                                      lane2_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice,
-                                      ctx->stream));
-    EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_nodes, 0, ne * sizeof(int32_t), ctx->stream));
-    EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_far, 0, ne * sizeof(double), ctx->stream));
-    EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_resc, 0, ne * sizeof(int32_t), ctx->stream));
+    for (int32_t w = 0; w < 4; ++w)
+        ctx->d_vjp_lists[w] = d_all_psi_tasks + vjp_at[w];
+    ctx->d_psi_tasks = d_all_psi_tasks + psi_at;
+    EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_far, 0, ne * (sizeof(double) + 2 * sizeof(int32_t)), ctx->stream));
     EPSEON_HIP_TRY(launch_shift_potential(ctx->stream, v_src, ctx->d_rec, count, max_table_chunks,
                                           ctx->d_ut, ctx->d_uv, ctx->d_uvr, d_edges));
     // Band windows: computed on the device, read back to size the segment
@@ -1256,61 +1271,85 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         if (ctx->wide_lanes == 0)
             jobs_wide.clear();
     }
-    // Windowed scan: work per task (trial energies times its band window's
-    // steps), its total, and its own XCD bins with the longest tasks first.
-    std::vector<double> band_task_work(scan_tasks.size());
-    for (size_t t = 0; t < scan_tasks.size(); ++t) {
-        const WaveTask& task = scan_tasks[t];
-        const PotentialRecord& r = ctx->rec[static_cast<size_t>(task.potential)];
-        const BandWindow& w = win_band[static_cast<size_t>(task.potential) * kBands +
-                                       static_cast<size_t>(host_group_band(r, task.first))];
-        band_task_work[t] = static_cast<double>(std::min(64, r.n_energies - task.first)) *
-                            static_cast<double>(w.hi - w.lo - 1);
-        scan_pu_band += band_task_work[t];
+    // Windowed scan: a task's work is its trial energies times its band
+    // window's steps.  Its own XCD bins, and within each chunk the longest
+    // tasks first: runs of equal work (a band's groups, the partly filled last
+    // group) by decreasing work.
+    std::vector<double> band_task_work(static_cast<size_t>(ctx->n_scan_tasks));
+    for (size_t k = 0; k < static_cast<size_t>(count); ++k) {
+        const PotentialRecord& r = rec_at(k);
+        const BandWindow* w = &win_band[static_cast<size_t>(order[k]) * kBands];
+        int32_t band = 0;
+        for (int32_t t = ctx->cum_scan_tasks[k], j = 0; t < ctx->cum_scan_tasks[k + 1]; ++t, j += 64) {
+            band = host_group_band(r, j, band);
+            const double x = static_cast<double>(std::min(64, r.n_energies - j)) *
+                             static_cast<double>(w[band].hi - w[band].lo - 1);
+            band_task_work[static_cast<size_t>(t)] = x;
+            scan_pu_band += x;
+        }
     }
     std::vector<int32_t> band_bins;
-    const std::vector<WaveTask> band_tasks =
-        xcd_binned(scan_tasks, ctx->cum_scan_tasks, band_task_work, true, band_bins, ctx->xcd_max_bin_band);
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(band_tasks.size(), 1), &ctx->d_xcd_scan_tasks_band));
-    EPSEON_HIP_TRY(arena_array(a, size_t(9), &ctx->d_xcd_bins_band));
-    if (!band_tasks.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_scan_tasks_band, band_tasks.data(),
-                                      band_tasks.size() * sizeof(WaveTask), hipMemcpyHostToDevice, ctx->stream));
-    EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_xcd_bins_band, band_bins.data(), 9 * sizeof(int32_t),
-                                  hipMemcpyHostToDevice, ctx->stream));
+    std::vector<TaskRun> band_runs;
+    {
+        struct Run {
+            int32_t i0, i1;
+            double work;
+        };
+        std::vector<Run> of_chunk;
+        int64_t at = 0;
+        const auto work = [&](size_t k, int32_t i0, int32_t i1) {
+            double sum = 0.0;
+            for (int32_t i = i0; i < i1; ++i)
+                sum += band_task_work[static_cast<size_t>(ctx->cum_scan_tasks[k] + i)];
+            return sum;
+        };
+        for (const TaskChunk& c : xcd_chunks(ctx->cum_scan_tasks, work, band_bins, ctx->xcd_max_bin_band)) {
+            const double* tw = &band_task_work[static_cast<size_t>(ctx->cum_scan_tasks[static_cast<size_t>(c.k)])];
+            of_chunk.clear();
+            for (int32_t i = c.i0; i < c.i1; ++i) {
+                if (of_chunk.empty() || of_chunk.back().work != tw[i])
+                    of_chunk.push_back({i, i, tw[i]});
+                of_chunk.back().i1 = i + 1;
+            }
+            std::stable_sort(of_chunk.begin(), of_chunk.end(),
+                             [](const Run& x, const Run& y) { return x.work > y.work; });
+            for (const Run& q : of_chunk) {
+                band_runs.push_back({at, order[static_cast<size_t>(c.k)], 64 * q.i0, 64, q.i1 - q.i0});
+                at += q.i1 - q.i0;
+            }
+        }
+    }
+    EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max(ctx->n_scan_tasks, 1)), &ctx->d_xcd_scan_tasks_band));
     ctx->scan_pu_band = scan_pu_band;
-    ctx->h_win_full = win_full;
-    ctx->h_win_band = win_band;
     ctx->segtab_ok = max_rows <= INT32_MAX / 512;
     EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(band_total, 1)) * 64, &ctx->d_segtab_band));
-    TableJob* d_jobs = nullptr;
-    EPSEON_HIP_TRY(arena_array(a, std::max<size_t>(jobs_full.size() + jobs_band.size() + jobs_wide.size(), 1), &d_jobs));
-    TableJob* d_jobs_wide = d_jobs + jobs_full.size() + jobs_band.size();
-    if (!jobs_wide.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_jobs_wide, jobs_wide.data(), jobs_wide.size() * sizeof(TableJob),
-                                      hipMemcpyHostToDevice, ctx->stream));
-    ctx->d_table_jobs = d_jobs;
     ctx->n_jobs_full = static_cast<int32_t>(jobs_full.size());
     ctx->n_jobs_band = static_cast<int32_t>(jobs_band.size());
     ctx->table_max_rows = max_rows;
     ctx->tables_full = ctx->tables_band = false;
-    if (count > 0) {
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_win_full, win_full.data(), win_full.size() * sizeof(BandWindow),
-                                      hipMemcpyHostToDevice, ctx->stream));
-        EPSEON_HIP_TRY(hipMemcpyAsync(ctx->d_win_band, win_band.data(), win_band.size() * sizeof(BandWindow),
-                                      hipMemcpyHostToDevice, ctx->stream));
+    // All table jobs in one array: whole grids, band windows, wide blocks.
+    std::vector<TableJob> jobs = std::move(jobs_full);
+    jobs.insert(jobs.end(), jobs_band.begin(), jobs_band.end());
+    jobs.insert(jobs.end(), jobs_wide.begin(), jobs_wide.end());
+    {
+        TaskRun* d_band_runs = nullptr;
+        Packed up(ctx->h_upload);
+        up.add(win_full, &ctx->d_win_full);
+        up.add(win_band, &ctx->d_win_band);
+        up.add(jobs, &ctx->d_table_jobs);
+        up.add(band_bins, &ctx->d_xcd_bins_band);
+        up.add(band_runs, &d_band_runs);
+        EPSEON_HIP_TRY(up.send(a, ctx->stream));
+        EPSEON_HIP_TRY(launch_task_lists(ctx->stream, d_band_runs, static_cast<int32_t>(band_runs.size()),
+                                         ctx->d_xcd_scan_tasks_band, nullptr, 0, nullptr));
     }
-    if (!jobs_full.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_jobs, jobs_full.data(), jobs_full.size() * sizeof(TableJob),
-                                      hipMemcpyHostToDevice, ctx->stream));
-    if (!jobs_band.empty())
-        EPSEON_HIP_TRY(hipMemcpyAsync(d_jobs + jobs_full.size(), jobs_band.data(),
-                                      jobs_band.size() * sizeof(TableJob), hipMemcpyHostToDevice,
-                                      ctx->stream));
+    ctx->h_win_full = std::move(win_full);
+    ctx->h_win_band = std::move(win_band);
+    const TableJob* d_jobs_wide = ctx->d_table_jobs + ctx->n_jobs_full + ctx->n_jobs_band;
     // The tables the current tuning's solve will use, built on stream2 while
     // the next scan runs; the refinement waits for them (tables_pending).
     const bool build_64 = mode_now == EPSEON_REFINE_SEGMENTED && lanes_now == 64 && ctx->segtab_ok &&
-                          jobs_full.size() + jobs_band.size() > 0;
+                          ctx->n_jobs_full + ctx->n_jobs_band > 0;
     if (build_64 || !jobs_wide.empty()) {
         EPSEON_HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
         EPSEON_HIP_TRY(hipStreamWaitEvent(ctx->stream2, ctx->ev_fork, 0));
@@ -1322,8 +1361,8 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         EPSEON_HIP_TRY(hipEventRecord(ctx->ev_tables, ctx->stream2));
         ctx->tables_pending = true;
     }
-    // The host buffers are pageable and owned by the caller: finish the
-    // copies before returning.
+    // The host buffers are pageable (V is the caller's): finish the copies
+    // before returning.
     EPSEON_HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->loaded = true;
     return EPSEON_OK;

@@ -2496,7 +2496,45 @@ __global__ __launch_bounds__(256) void bracket_kernel(const PotentialRecord* __r
                                  rescales, points[out]);
 }
 
+// Task lists from their runs, one wavefront per run.
+__global__ __launch_bounds__(256) void task_list_kernel(const TaskRun* __restrict__ runs, const int32_t n_runs,
+                                                        WaveTask* __restrict__ out)
+{
+    const int32_t r = wave_task_index();
+    if (r >= n_runs)
+        return;
+    const TaskRun R = runs[r];
+    for (int32_t i = static_cast<int32_t>(threadIdx.x & 63); i < R.count; i += 64)
+        out[R.out + i] = WaveTask{R.potential, R.first + i * R.step};
+}
+
+__global__ __launch_bounds__(256) void psi_list_kernel(const PsiRun* __restrict__ runs, const int32_t n_runs,
+                                                       PsiTask* __restrict__ out)
+{
+    const int32_t r = wave_task_index();
+    if (r >= n_runs)
+        return;
+    const PsiRun R = runs[r];
+    for (int32_t i = static_cast<int32_t>(threadIdx.x & 63); i < R.segs * R.groups; i += 64)
+        out[R.out + i] = PsiTask{R.potential, 64 * (i % R.groups), R.side, i / R.groups};
+}
+
 // ---------------------------------------------------------------- launchers
+
+hipError_t launch_task_lists(hipStream_t stream, const TaskRun* runs, int32_t n_runs, WaveTask* tasks,
+                             const PsiRun* psi_runs, int32_t n_psi_runs, PsiTask* psi_tasks)
+{
+    if (n_runs > 0) {
+        hipLaunchKernelGGL(task_list_kernel, dim3(static_cast<unsigned>((n_runs + 3) / 4)), dim3(256), 0, stream, runs,
+                           n_runs, tasks);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess)
+            return e;
+    }
+    if (n_psi_runs > 0)
+        hipLaunchKernelGGL(psi_list_kernel, dim3(static_cast<unsigned>((n_psi_runs + 3) / 4)), dim3(256), 0, stream,
+                           psi_runs, n_psi_runs, psi_tasks);
+    return hipGetLastError();
+}
 
 // chunk0[p]: the number of chunks of the potentials before p; max_chunks: the
 // most of one potential.

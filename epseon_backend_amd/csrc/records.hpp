@@ -271,4 +271,18 @@ struct WaveTask {
     int32_t first;
 };
 
+// Consecutive tasks of a list, written on the device: entries out .. out +
+// count - 1 are (potential, first + i step).
+struct TaskRun {
+    int64_t out;
+    int32_t potential, first, step, count;
+};
+
+// The eigenfunction tasks of one side of a potential: for each of `segs`
+// segments, `groups` groups of 64 levels.
+struct PsiRun {
+    int64_t out;
+    int32_t potential, side, segs, groups;
+};
+
 }  // namespace epseon::hip
