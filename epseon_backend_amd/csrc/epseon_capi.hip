@@ -31,7 +31,7 @@ hipError_t launch_shift_potential(hipStream_t, const double*, const PotentialRec
 hipError_t launch_potential_stats(hipStream_t, const double*, const int64_t*, const int64_t*, const int32_t*,
                                   const double*, int32_t, int32_t, ChunkMin*, PotentialStats*);
 hipError_t launch_scan(hipStream_t, const double*, const PotentialRecord*, const BandWindow*,
-                       const WaveTask*, int32_t, const int32_t*, int32_t, int32_t, int32_t*, double*,
+                       const WaveTask*, int32_t, const int32_t*, int32_t, int32_t, int32_t, int32_t*, double*,
                        int32_t*);
 hipError_t launch_brackets(hipStream_t, const PotentialRecord*, const BandWindow*, const WaveTask*, int32_t,
                            const int32_t*, const double*, const int32_t*, Bracket*, RefinePoints*);
@@ -183,6 +183,11 @@ constexpr int32_t kWideTableMinPoints = 16384;
 // host walk takes 0.65 ns a point, the two passes and their read-back 50 us
 // and little more.
 constexpr int64_t kDeviceStatsMinPoints = 100000;
+
+// Scans of at most this many wavefronts per SIMD, of whole grids or of at least
+// this many steps on average, spread over the SIMDs as scan_shape says.
+constexpr int64_t kSpreadMaxScanWavesPerSimd = 48;
+constexpr double kSpreadMinSteps = 4096.0;
 
 // Automatic windows need at least this many scan wavefronts per SIMD.
 constexpr int64_t kWindowsMinScanWavesPerSimd = 8;
@@ -1470,18 +1475,31 @@ const BandWindow* scan_window_set(const epseon_ctx* ctx)
     return ctx->scan_windows ? ctx->d_win_band : ctx->d_win_full;
 }
 
-// Wavefronts per scan workgroup.  Whole-grid scans with at most a few
-// wavefronts per SIMD take their time from the fullest SIMD, and one-wavefront
-// workgroups pile up on some SIMDs depending on what ran before; workgroups of
-// four put one wavefront on each SIMD of a compute unit.  Measured on 8 x
-// 200,000 points x 16,384 energies (two wavefronts per SIMD) after a load:
-// 4.9 -> 3.3 ms per scan; with one per SIMD or less within 2 %.  Longer scans
-// (and windowed ones, whose wavefronts differ) keep the tuning's value: the
-// SIMDs take new wavefronts as others end.
-int32_t scan_waves_per_block(const epseon_ctx* ctx)
+// Wavefronts and LDS bytes per scan workgroup.  With up to a few tens of
+// wavefronts per SIMD the scan ends when its fullest SIMD does.  If all of
+// them may be resident, each SIMD gets its share at once, long and short
+// windows as they come, and one-wavefront workgroups also pile up on some
+// SIMDs depending on what ran before.  Workgroups of four put one wavefront on
+// each SIMD of a compute unit, and 60 KB of LDS, which nothing uses, let two of
+// them run there at a time (and leave room for a workgroup of the segment
+// tables beside them): enough to fill the issue slots, and the rest goes to
+// the SIMDs that come free.  Measured, tuning's value against this one:
+// 8.8 wavefronts per SIMD (256 ragged potentials) 0.94 and 0.76 ms, 8.0 (512 x
+// 50,000 points) 2.78 and 2.32, 18 (512 ragged) 1.60 and 1.31, 37 (1,024) 3.05
+// and 2.94, 72 (2,048) 5.57 and 5.68; whole grids, 5.1 per SIMD 1.05 and 0.88,
+// one 1.73 and 1.69.  Windowed shots of 1,500 steps lose (0.30 and 0.33 ms): a
+// workgroup holds its place until its longest wavefront ends.
+struct ScanShape {
+    int32_t waves, lds;
+};
+
+ScanShape scan_shape(const epseon_ctx* ctx)
 {
-    const bool few = static_cast<int64_t>(ctx->n_scan_tasks) < kWindowsMinScanWavesPerSimd * 4 * ctx->compute_units;
-    return ctx->waves_per_block == 1 && !ctx->scan_windows && few ? 4 : ctx->waves_per_block;
+    const int64_t simds = 4 * static_cast<int64_t>(ctx->compute_units);
+    const double steps = ctx->scan_point_updates / (64.0 * std::max(ctx->n_scan_tasks, 1));
+    const bool spread = ctx->waves_per_block == 1 && ctx->n_scan_tasks <= kSpreadMaxScanWavesPerSimd * simds &&
+                        (!ctx->scan_windows || steps >= kSpreadMinSteps);
+    return spread ? ScanShape{4, 60 << 10} : ScanShape{ctx->waves_per_block, 0};
 }
 
 // Scan of the potentials [k0, k1) in task order on `stream`; the whole batch
@@ -1491,18 +1509,18 @@ hipError_t run_scan(epseon_ctx* ctx, hipStream_t stream, size_t k0, size_t k1)
     const int32_t t0 = ctx->cum_scan_tasks[k0];
     const int32_t t1 = ctx->cum_scan_tasks[k1];
     const BandWindow* win = scan_window_set(ctx);
-    const int32_t waves = scan_waves_per_block(ctx);
+    const ScanShape shape = scan_shape(ctx);
     if (ctx->xcd_scan && k0 == 0 && k1 == ctx->cum_scan_tasks.size() - 1) {
         if (ctx->scan_windows)
             return launch_scan(stream, ctx->d_ut, ctx->d_rec, win, ctx->d_xcd_scan_tasks_band, t1 - t0,
-                               ctx->d_xcd_bins_band, ctx->xcd_max_bin_band, waves,
+                               ctx->d_xcd_bins_band, ctx->xcd_max_bin_band, shape.waves, shape.lds,
                                ctx->d_nodes, ctx->d_far, ctx->d_resc);
         return launch_scan(stream, ctx->d_ut, ctx->d_rec, win, ctx->d_xcd_scan_tasks, t1 - t0,
-                           ctx->d_xcd_bins, ctx->xcd_max_bin, waves, ctx->d_nodes,
+                           ctx->d_xcd_bins, ctx->xcd_max_bin, shape.waves, shape.lds, ctx->d_nodes,
                            ctx->d_far, ctx->d_resc);
     }
     return launch_scan(stream, ctx->d_ut, ctx->d_rec, win, ctx->d_scan_tasks + t0, t1 - t0, nullptr, 0,
-                       waves, ctx->d_nodes, ctx->d_far, ctx->d_resc);
+                       shape.waves, shape.lds, ctx->d_nodes, ctx->d_far, ctx->d_resc);
 }
 
 // Make `stream` wait for the segment tables of the last load (once), and,

@@ -2571,9 +2571,10 @@ hipError_t launch_shift_potential(hipStream_t stream, const double* v, const Pot
 
 // bins == nullptr: tasks[0, n_tasks) in order.  Otherwise `bins` (device, 9
 // offsets) splits the list per XCD and `max_bin` is the largest bin's size.
+// `lds` bytes of dynamic LDS per workgroup limit how many share a compute unit.
 hipError_t launch_scan(hipStream_t stream, const double* ut, const PotentialRecord* pots,
                        const BandWindow* windows, const WaveTask* tasks, int32_t n_tasks,
-                       const int32_t* bins, int32_t max_bin, int32_t waves_per_block, int32_t* nodes,
+                       const int32_t* bins, int32_t max_bin, int32_t waves_per_block, int32_t lds, int32_t* nodes,
                        double* far_end, int32_t* rescales)
 {
     if (n_tasks == 0)
@@ -2581,8 +2582,8 @@ hipError_t launch_scan(hipStream_t stream, const double* ut, const PotentialReco
     const int32_t blocks = bins == nullptr ? (n_tasks + waves_per_block - 1) / waves_per_block
                                            : 8 * ((max_bin + waves_per_block - 1) / waves_per_block);
     hipLaunchKernelGGL(numerov_scan_kernel, dim3(static_cast<unsigned>(blocks)),
-                       dim3(static_cast<unsigned>(64 * waves_per_block)), 0, stream, ut, pots, windows,
-                       tasks, n_tasks, bins, nodes, far_end, rescales);
+                       dim3(static_cast<unsigned>(64 * waves_per_block)), static_cast<unsigned>(lds), stream, ut, pots,
+                       windows, tasks, n_tasks, bins, nodes, far_end, rescales);
     return hipGetLastError();
 }
 
