@@ -144,8 +144,19 @@ constexpr int32_t psi_short_seg_len(const int32_t n_points)
     return 32 * b < most ? 32 * b : most;
 }
 
+// The segments of a side's shot (side 0: from the left wall, points
+// first_point + 1 upwards; 1: from the right wall downwards) start psi_shift
+// steps before the multiples of psi_seg_len, so that from the second segment
+// on a 32-step block writes 32 values that start at a multiple of 16 of the
+// untrimmed grid: whole 128-byte lines wherever rows start at one.  The last
+// segment ends with the shot.
+constexpr int32_t psi_shift(const int64_t first_point, const int32_t n_points, const int32_t side)
+{
+    return static_cast<int32_t>((side == 0 ? first_point + 1 : -(first_point + n_points - 1)) & 15);
+}
+
 // State of an eigenfunction shot at the start of one of its segments (after
-// j = segment * psi_seg_len steps): y_{j+1}, y_j and their difference as
+// j = segment * psi_seg_len - psi_shift steps): y_{j+1}, y_j and their difference as
 // mantissas of the binary exponent k (the true values are these times 2^k).
 // f and f_prev are recomputed from the table.
 struct alignas(32) PsiCheckpoint {
