@@ -34,7 +34,7 @@ hipError_t launch_scan(hipStream_t, const double*, const PotentialRecord*, const
                        const WaveTask*, int32_t, const int32_t*, int32_t, int32_t, int32_t, int32_t*, double*,
                        int32_t*);
 hipError_t launch_brackets(hipStream_t, const PotentialRecord*, const BandWindow*, const WaveTask*, int32_t,
-                           const int32_t*, const double*, const int32_t*, Bracket*, RefinePoints*);
+                           const int32_t*, const double*, const int32_t*, Bracket*, RefinePoints*, int64_t*);
 hipError_t launch_refine(hipStream_t, int32_t, const double*, const PotentialRecord*, const BandWindow*,
                          const WaveTask*, int32_t, int32_t, const Bracket*, RefinePoints*, double, int32_t,
                          double*, int32_t*, int32_t*, int32_t*);
@@ -47,8 +47,8 @@ hipError_t launch_segment_tables(hipStream_t, const double*, const PotentialReco
 hipError_t launch_task_lists(hipStream_t, const TaskRun*, int32_t, WaveTask*, const PsiRun*, int32_t, PsiTask*);
 hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord*, int32_t, int64_t,
                                const ChunkEdge*, int2*);
-hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, int32_t, const int32_t*, const int32_t*,
-                                const int32_t*, int64_t*);
+hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, const WaveTask*, int32_t, const int32_t*,
+                                const int32_t*, const int32_t*, int64_t*);
 hipError_t launch_normalize(hipStream_t, const double*, const double*, const PotentialRecord*,
                             const PsiTask*, int32_t, const WaveTask*, int32_t, const double*, const int32_t*,
                             PsiSegMatrix*, PsiCheckpoint*, LevelNorm*);
@@ -1551,7 +1551,7 @@ hipError_t run_refine(epseon_ctx* ctx, hipStream_t stream, hipStream_t stream_b,
     const int32_t t1 = ctx->cum_level_tasks[k1];
     if (const hipError_t e = launch_brackets(stream, ctx->d_rec, win, ctx->d_level_tasks + t0, t1 - t0,
                                              ctx->d_nodes, ctx->d_far, ctx->d_resc, ctx->d_brackets,
-                                             ctx->d_points);
+                                             ctx->d_points, ctx->d_summary);
         e != hipSuccess)
         return e;
     if (mode == EPSEON_REFINE_LANE && ctx->levels_per_lane == 1) {
@@ -1644,7 +1644,7 @@ size_t split_point(const epseon_ctx* ctx, double fraction)
 // every refinement (outside any recorded graph).
 hipError_t enqueue_summary(epseon_ctx* ctx)
 {
-    return launch_level_summary(ctx->stream, ctx->d_rec, static_cast<int32_t>(ctx->rec.size()), ctx->d_status,
+    return launch_level_summary(ctx->stream, ctx->d_rec, ctx->d_level_tasks, ctx->n_level_tasks, ctx->d_status,
                                 ctx->d_iters, ctx->d_steps, ctx->d_summary);
 }
 

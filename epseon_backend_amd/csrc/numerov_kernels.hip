@@ -1035,116 +1035,138 @@ __device__ __forceinline__ void model_apply(const double b, const double e0, con
     k = k + n;
 }
 
-// Bracket of level v from the scan: the first trial energy with more than v
-// nodes and the one below it (or the window floor, below which no level
-// exists since every eigenvalue exceeds min V).  Exponents are binary.  When
-// the bracket holds exactly level v and a third scan point of the same count
-// regime exists above or below it, `rate` is the model rate b.  `pts` gets
-// the level's interpolation points: scan points j - kPts/2 .. j + kPts/2 - 1
-// (j the upper end) whose group shares the level's window, the lower end only
-// when its value is of that window.
-// W: the potential's kBands band windows (those the scan used).
-__device__ __forceinline__ Bracket find_bracket(const PotentialRecord& P, const BandWindow* W,
-                                                const int32_t v, const int32_t* __restrict__ nodes,
-                                                const double* __restrict__ far_end,
-                                                const int32_t* __restrict__ rescales, RefinePoints& pts)
+// Value of row lane `from` of this lane's 16-lane row.
+template <class V>
+__device__ __forceinline__ V row_value(const V x, const int32_t from)
 {
-    Bracket b{};
-    pts.n = 0;
-    pts.ih = 0;
+    return __shfl(x, from, 16);
+}
+
+// The row's 16 bits of a ballot.
+__device__ __forceinline__ uint32_t row_ballot(const bool x)
+{
+    return static_cast<uint32_t>(__ballot(x) >> (threadIdx.x & 48)) & 0xFFFFu;
+}
+
+// Bracket of level v from the scan, by a 16-lane row (lane i of it): the first
+// trial energy j with more than v nodes and the one below it (or the window
+// floor, below which no level exists since every eigenvalue exceeds min V).
+// Exponents are binary.  When the bracket holds exactly level v and a third
+// scan point of the same count regime exists above or below it, `rate` is the
+// model rate b.  `pts` gets the level's interpolation points: scan points j -
+// kPts/2 .. j + kPts/2 - 1 whose group shares the level's window, the lower end
+// only when its value is of that window.
+// The search for j is a binary one whose next four steps are loaded at once
+// (lane i holds node i of their decision tree), and lane s loads candidate
+// point s: a handful of dependent loads, where one lane per level made a dozen
+// for the search alone (17 levels: 15 -> 6.4 us; 4,096 potentials of 24
+// levels: 104 -> 120 us of 17 ms, as it loads more lines).
+// W: the potential's kBands band windows (those the scan used).
+__device__ __forceinline__ void find_bracket(const PotentialRecord& P, const BandWindow* W, const int32_t v,
+                                             const int32_t i, const int32_t* __restrict__ nodes,
+                                             const double* __restrict__ far_end,
+                                             const int32_t* __restrict__ rescales, Bracket& out, RefinePoints& pts)
+{
+    static_assert(kPts <= 16, "a lane per candidate point");
+    constexpr int32_t kUp = kPts / 2;  // the lane of point j
     const int32_t m = P.n_energies;
     const int32_t* nd = nodes + P.energy_offset;
     int32_t lo = 0, hi = m;
     while (lo < hi) {
-        const int32_t mid = (lo + hi) >> 1;
-        if (nd[mid] > v)
-            hi = mid;
-        else
-            lo = mid + 1;
+        int32_t l = lo, h = hi;
+        for (int32_t b = 30 - __builtin_clz(i | 1); b >= 0; --b)
+            if (l < h) {
+                const int32_t mid = (l + h) >> 1;
+                if ((i >> b) & 1)
+                    l = mid + 1;
+                else
+                    h = mid;
+            }
+        const uint32_t over = row_ballot(i > 0 && l < h && nd[(l + h) >> 1] > v);
+        int32_t node = 1;
+#pragma unroll
+        for (int32_t d = 0; d < 4; ++d)
+            if (lo < hi) {
+                const int32_t mid = (lo + hi) >> 1;
+                const int32_t right = (over >> node) & 1u ? 0 : 1;
+                if (right)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+                node = 2 * node + right;
+            }
     }
     const int32_t j = lo;
     if (j == m) {
-        b.found = 0;
-        return b;
+        if (i == 0) {
+            out = Bracket{};
+            pts.n = 0;
+            pts.ih = 0;
+        }
+        return;
     }
-    const int32_t band = group_band(P, j);
-    const int32_t fe = W[band].far_exp;
+    // Lane i's candidate point.
+    const int32_t q = j - kUp + i;
+    const bool in = i < kPts && q >= 0 && q < m;
+    int32_t bq = 0, c = 0, k = 0;
+    double w = 0.0;
+    if (in) {
+        const int64_t o = P.energy_offset + q;
+        bq = group_band(P, q);
+        c = nd[q];
+        w = far_end[o];
+        k = W[bq].far_exp - rescales[o] * kRescaleLog2;
+    }
+    const int32_t band = row_value(bq, kUp);
+    const bool same = in && same_window(W, bq, band);
+    // Every count before j is at most v.
+    const bool lo_ok = j > 0;
+    const bool lo_foreign = lo_ok && !row_value(static_cast<int32_t>(same), kUp - 1);
+    const double e = __builtin_fma(static_cast<double>(q + 1), P.de, P.e_lo);
+    // The points, compacted; the slots past them are zero.
+    const uint32_t ok = row_ballot(same);
+    const int32_t n = __builtin_popcount(ok);
+    const int32_t before = __builtin_popcount(ok & ((1u << i) - 1u));
+    if (i < kPts) {
+        const int32_t slot = same ? before : n + i - before;
+        pts.e[slot] = same ? e : 0.0;
+        pts.w[slot] = same ? w : 0.0;
+        pts.k[slot] = same ? k : 0;
+    }
+    const double wl = row_value(w, kUp - 1), wh = row_value(w, kUp);
+    const int32_t kl = row_value(k, kUp - 1), kh = row_value(k, kUp);
+    const int32_t cl = row_value(c, kUp - 1), ch = row_value(c, kUp);
+    // The third point of the rate: the one above when it has the upper end's
+    // count, else the one below the lower end with its count.
+    const uint32_t regime = row_ballot(same && ((i == kUp + 1 && c == ch) || (i == kUp - 2 && c == cl)));
+    const bool above = (regime >> (kUp + 1)) & 1u;
+    const int32_t third = above ? kUp + 1 : kUp - 2;
+    const double wt = row_value(w, third);
+    const int32_t kt = row_value(k, third);
+    if (i != 0)
+        return;
+    pts.n = n;
+    pts.ih = __builtin_popcount(ok & ((1u << kUp) - 1u));
+    Bracket b{};
     b.found = 1;
     b.band = band;
     b.eh = __builtin_fma(static_cast<double>(j + 1), P.de, P.e_lo);
-    b.ch = nd[j];
-    b.wh = far_end[P.energy_offset + j];
-    b.kh = fe - rescales[P.energy_offset + j] * kRescaleLog2;
-    if (j == 0 || nd[j - 1] > v) {
-        b.el = P.e_lo;
-        b.cl = 0;
-        b.lo_ok = 0;
-    } else {
-        const int32_t bl = group_band(P, j - 1);
+    b.ch = ch;
+    b.wh = wh;
+    b.kh = kh;
+    b.el = P.e_lo;
+    if (lo_ok) {
         b.el = __builtin_fma(static_cast<double>(j), P.de, P.e_lo);
-        b.cl = nd[j - 1];
-        b.wl = far_end[P.energy_offset + j - 1];
-        b.kl = W[bl].far_exp - rescales[P.energy_offset + j - 1] * kRescaleLog2;
+        b.cl = cl;
+        b.wl = wl;
+        b.kl = kl;
         b.lo_ok = 1;
-        b.lo_foreign = same_window(W, bl, band) ? 0 : 1;
+        b.lo_foreign = lo_foreign ? 1 : 0;
+        if (!lo_foreign && cl == v && ch == v + 1 && regime != 0)
+            b.rate = above ? model_rate(wl, kl, wh, kh, wt, kt, true, P.de)
+                           : model_rate(wt, kt, wl, kl, wh, kh, false, P.de);
     }
-    // Candidates j - kPts/2 + s, compacted in registers (every slot addressed
-    // by a constant index), then the record is written whole.
-    double pe[kPts], pw[kPts];
-    int32_t pk[kPts];
-    int32_t np = 0, ih = 0;
-#pragma unroll
-    for (int32_t s = 0; s < kPts; ++s) {
-        pe[s] = 0.0;
-        pw[s] = 0.0;
-        pk[s] = 0;
-    }
-#pragma unroll
-    for (int32_t s = 0; s < kPts; ++s) {
-        const int32_t q = j - kPts / 2 + s;
-        bool ok = q >= 0 && q < m;
-        int32_t bq = band;
-        if (ok && q == j - 1)
-            ok = b.lo_ok && !b.lo_foreign;
-        else if (ok && q != j) {
-            bq = group_band(P, q);
-            ok = same_window(W, bq, band);
-        }
-        if (ok) {
-            const double e = __builtin_fma(static_cast<double>(q + 1), P.de, P.e_lo);
-            const double w = far_end[P.energy_offset + q];
-            const int32_t k = W[bq].far_exp - rescales[P.energy_offset + q] * kRescaleLog2;
-#pragma unroll
-            for (int32_t t = 0; t < kPts; ++t)
-                if (t == np) {
-                    pe[t] = e;
-                    pw[t] = w;
-                    pk[t] = k;
-                }
-            if (q == j)
-                ih = np;
-            ++np;
-        }
-    }
-#pragma unroll
-    for (int32_t t = 0; t < kPts; ++t) {
-        pts.e[t] = pe[t];
-        pts.w[t] = pw[t];
-        pts.k[t] = pk[t];
-    }
-    pts.n = np;
-    pts.ih = ih;
-    b.rate = 0.0;
-    if (b.lo_ok && !b.lo_foreign && b.cl == v && b.ch == v + 1) {
-        const int64_t o = P.energy_offset;
-        if (j + 1 < m && nd[j + 1] == b.ch && same_window(W, group_band(P, j + 1), band))
-            b.rate = model_rate(b.wl, b.kl, b.wh, b.kh, far_end[o + j + 1],
-                                fe - rescales[o + j + 1] * kRescaleLog2, true, P.de);
-        else if (j >= 2 && nd[j - 2] == b.cl && same_window(W, group_band(P, j - 2), band))
-            b.rate = model_rate(far_end[o + j - 2], fe - rescales[o + j - 2] * kRescaleLog2, b.wl, b.kl,
-                                b.wh, b.kh, false, P.de);
-    }
-    return b;
+    out = b;
 }
 
 // Insert a shot at em (inside the bracket: at index ih in energy order).  A
@@ -2480,10 +2502,9 @@ numerov_refine_segmented_kernel(const double* __restrict__ uv, const double* __r
     }
 }
 
-// Bracket pass: one thread per level task (potential, level index) finds
-// the level's bracket in the scan arrays (binary search over its
-// potential's node counts, model rate from three scan points), so the
-// refinement's wavefronts start shooting at once.
+// Bracket pass: a 16-lane row per level task (potential, level index) finds
+// the level's bracket in the scan arrays, so the refinement's wavefronts start
+// shooting at once.  Also clears the summary that follows the refinement.
 __global__ __launch_bounds__(256) void bracket_kernel(const PotentialRecord* __restrict__ pots,
                                                       const BandWindow* __restrict__ windows,
                                                       const WaveTask* __restrict__ tasks, const int32_t n_tasks,
@@ -2491,9 +2512,12 @@ __global__ __launch_bounds__(256) void bracket_kernel(const PotentialRecord* __r
                                                       const double* __restrict__ far_end,
                                                       const int32_t* __restrict__ rescales,
                                                       Bracket* __restrict__ brackets,
-                                                      RefinePoints* __restrict__ points)
+                                                      RefinePoints* __restrict__ points,
+                                                      unsigned long long* __restrict__ summary)
 {
-    const int32_t t = static_cast<int32_t>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (blockIdx.x == 0 && threadIdx.x < 3)
+        summary[threadIdx.x] = 0;
+    const int32_t t = static_cast<int32_t>(blockIdx.x * 16 + threadIdx.x / 16);
     if (t >= n_tasks)
         return;
     const WaveTask task = tasks[t];
@@ -2501,8 +2525,8 @@ __global__ __launch_bounds__(256) void bracket_kernel(const PotentialRecord* __r
     if (P.flags != 0 || task.first >= P.level_count)
         return;
     const int64_t out = P.level_offset + task.first;
-    brackets[out] = find_bracket(P, windows + task.potential * kBands, P.level_min + task.first, nodes, far_end,
-                                 rescales, points[out]);
+    find_bracket(P, windows + task.potential * kBands, P.level_min + task.first,
+                 static_cast<int32_t>(threadIdx.x % 16), nodes, far_end, rescales, brackets[out], points[out]);
 }
 
 // Task lists from their runs, one wavefront per run.
@@ -2599,12 +2623,13 @@ hipError_t launch_scan(hipStream_t stream, const double* ut, const PotentialReco
 hipError_t launch_brackets(hipStream_t stream, const PotentialRecord* pots, const BandWindow* windows,
                            const WaveTask* level_tasks, int32_t n_tasks, const int32_t* nodes,
                            const double* far_end, const int32_t* rescales, Bracket* brackets,
-                           RefinePoints* points)
+                           RefinePoints* points, int64_t* summary)
 {
     if (n_tasks == 0)
         return hipSuccess;
-    hipLaunchKernelGGL(bracket_kernel, dim3(static_cast<unsigned>((n_tasks + 255) / 256)), dim3(256), 0, stream,
-                       pots, windows, level_tasks, n_tasks, nodes, far_end, rescales, brackets, points);
+    hipLaunchKernelGGL(bracket_kernel, dim3(static_cast<unsigned>((n_tasks + 15) / 16)), dim3(256), 0, stream, pots,
+                       windows, level_tasks, n_tasks, nodes, far_end, rescales, brackets, points,
+                       reinterpret_cast<unsigned long long*>(summary));
     return hipGetLastError();
 }
 
@@ -2701,60 +2726,63 @@ hipError_t launch_segment_tables(hipStream_t stream, const double* uv, const Pot
     return hipGetLastError();
 }
 
-// Refinement summary for the statistics, one wavefront per kSummaryPots
-// potentials adding its sums to out (zeroed first): out[0] = sum of
-// iterations x steps over levels that shot, out[1] = converged levels,
-// out[2] = sum over converged levels of their grid's n - 2 steps.  Integer
-// sums, so the result does not depend on the order.
-constexpr int32_t kSummaryPots = 16;
-__global__ __launch_bounds__(64) void level_summary_kernel(const PotentialRecord* __restrict__ pots,
-                                                           const int32_t n_pots, const int32_t* __restrict__ status,
-                                                           const int32_t* __restrict__ iterations,
-                                                           const int32_t* __restrict__ steps,
-                                                           unsigned long long* __restrict__ out)
+// Refinement summary for the statistics, from the level tasks: out[0] += sum
+// of iterations x steps over levels that shot, out[1] += converged levels,
+// out[2] += sum over converged levels of their grid's n - 2 steps (cleared by
+// the bracket pass).  Integer sums, so the result does not depend on the order.
+// One atomic per sum and workgroup of kSummaryLevels levels (98,304 levels:
+// 13.6 us, where a wavefront per few potentials took 51 us).
+constexpr int32_t kSummaryLevels = 1024;
+__global__ __launch_bounds__(256) void level_summary_kernel(const PotentialRecord* __restrict__ pots,
+                                                            const WaveTask* __restrict__ tasks, const int32_t n_tasks,
+                                                            const int32_t* __restrict__ status,
+                                                            const int32_t* __restrict__ iterations,
+                                                            const int32_t* __restrict__ steps,
+                                                            unsigned long long* __restrict__ out)
 {
-    const int32_t p0 = static_cast<int32_t>(blockIdx.x) * kSummaryPots;
-    const int32_t p1 = min(n_pots, p0 + kSummaryPots);
+    __shared__ int64_t s_sum[4][3];
+    const int32_t t0 = static_cast<int32_t>(blockIdx.x) * kSummaryLevels;
+    const int32_t t1 = min(n_tasks, t0 + kSummaryLevels);
     int64_t sum[3] = {0, 0, 0};
-    for (int32_t p = p0; p < p1; ++p) {
-        const PotentialRecord& r = pots[p];
-        for (int32_t l = static_cast<int32_t>(threadIdx.x); l < r.level_count; l += 64) {
-            const int64_t o = r.level_offset + l;
-            const int32_t it = iterations[o];
-            if (it > 0)
-                sum[0] += static_cast<int64_t>(it) * steps[o];
-            if (status[o] == 0) {
-                sum[1] += 1;
-                sum[2] += r.n_points - 2;
-            }
+    for (int32_t t = t0 + static_cast<int32_t>(threadIdx.x); t < t1; t += 256) {
+        const WaveTask task = tasks[t];
+        const PotentialRecord& P = pots[task.potential];
+        const int64_t o = P.level_offset + task.first;
+        const int32_t it = iterations[o];
+        if (it > 0)
+            sum[0] += static_cast<int64_t>(it) * steps[o];
+        if (status[o] == 0) {
+            sum[1] += 1;
+            sum[2] += P.n_points - 2;
         }
     }
 #pragma unroll
     for (int32_t q = 0; q < 3; ++q) {
-        int64_t x = sum[q];
 #pragma unroll
         for (int32_t d = 32; d >= 1; d /= 2)
-            x += __shfl_xor(x, d, 64);
-        if (threadIdx.x == 0 && x != 0)
+            sum[q] += __shfl_xor(sum[q], d, 64);
+        if ((threadIdx.x & 63) == 0)
+            s_sum[threadIdx.x >> 6][q] = sum[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        const int32_t q = static_cast<int32_t>(threadIdx.x);
+        const int64_t x = s_sum[0][q] + s_sum[1][q] + s_sum[2][q] + s_sum[3][q];
+        if (x != 0)
             atomicAdd(out + q, static_cast<unsigned long long>(x));
     }
 }
 
-__global__ void zero_summary_kernel(unsigned long long* __restrict__ out)
+hipError_t launch_level_summary(hipStream_t stream, const PotentialRecord* pots, const WaveTask* level_tasks,
+                                int32_t n_tasks, const int32_t* status, const int32_t* iterations,
+                                const int32_t* steps, int64_t* out)
 {
-    if (threadIdx.x < 3)
-        out[threadIdx.x] = 0;
-}
-
-hipError_t launch_level_summary(hipStream_t stream, const PotentialRecord* pots, int32_t n_pots,
-                                const int32_t* status, const int32_t* iterations, const int32_t* steps,
-                                int64_t* out)
-{
-    unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
-    hipLaunchKernelGGL(zero_summary_kernel, dim3(1), dim3(64), 0, stream, o);
-    if (n_pots > 0)
-        hipLaunchKernelGGL(level_summary_kernel, dim3(static_cast<unsigned>((n_pots + kSummaryPots - 1) / kSummaryPots)),
-                           dim3(64), 0, stream, pots, n_pots, status, iterations, steps, o);
+    if (n_tasks == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(level_summary_kernel,
+                       dim3(static_cast<unsigned>((n_tasks + kSummaryLevels - 1) / kSummaryLevels)), dim3(256), 0,
+                       stream, pots, level_tasks, n_tasks, status, iterations, steps,
+                       reinterpret_cast<unsigned long long*>(out));
     return hipGetLastError();
 }
 
