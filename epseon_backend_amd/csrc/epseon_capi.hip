@@ -44,7 +44,8 @@ hipError_t launch_refine_segmented(hipStream_t, int32_t, int32_t, const double*,
                                    double*, int32_t*, int32_t*, int32_t*);
 hipError_t launch_segment_tables(hipStream_t, const double*, const PotentialRecord*, const TableJob*,
                                  int32_t, int32_t, int32_t, double*);
-hipError_t launch_task_lists(hipStream_t, const TaskRun*, int32_t, WaveTask*, const PsiRun*, int32_t, PsiTask*);
+hipError_t launch_load_lists(hipStream_t, const TaskRun*, int32_t, WaveTask*, const PsiRun*, int32_t, PsiTask*, void*,
+                             int64_t);
 hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord*, int32_t, int64_t,
                                const ChunkEdge*, int2*);
 hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, const WaveTask*, int32_t, const int32_t*,
@@ -1161,9 +1162,9 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     }
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_norms));
     EPSEON_HIP_TRY(arena_array(a, nl, &ctx->d_grad_levels));
+    TaskRun* d_runs = nullptr;
+    PsiRun* d_psi_runs = nullptr;
     {
-        TaskRun* d_runs = nullptr;
-        PsiRun* d_psi_runs = nullptr;
         Packed up(ctx->h_upload);
         up.add(ctx->rec, &ctx->d_rec);
         up.add(runs, &d_runs);
@@ -1173,8 +1174,6 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         for (int32_t g = 0; g < 2; ++g)
             up.add(xcd_group_bins[g], &ctx->d_xcd_group_bins[g]);
         EPSEON_HIP_TRY(up.send(a, ctx->stream));
-        EPSEON_HIP_TRY(launch_task_lists(ctx->stream, d_runs, static_cast<int32_t>(runs.size()), d_wave_tasks,
-                                         d_psi_runs, static_cast<int32_t>(psi_runs.size()), d_all_psi_tasks));
     }
     ctx->d_scan_tasks = d_wave_tasks + scan_at;
     ctx->d_refine_tasks = d_wave_tasks + refine_at;
@@ -1190,7 +1189,6 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     for (int32_t w = 0; w < 4; ++w)
         ctx->d_vjp_lists[w] = d_all_psi_tasks + vjp_at[w];
     ctx->d_psi_tasks = d_all_psi_tasks + psi_at;
-    EPSEON_HIP_TRY(hipMemsetAsync(ctx->d_far, 0, ne * (sizeof(double) + 2 * sizeof(int32_t)), ctx->stream));
     EPSEON_HIP_TRY(launch_shift_potential(ctx->stream, v_src, ctx->d_rec, count, max_table_chunks,
                                           ctx->d_ut, ctx->d_uv, ctx->d_uvr, d_edges));
     // Band windows: computed on the device, read back to size the segment
@@ -1202,6 +1200,12 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         EPSEON_HIP_TRY(hipMemcpyAsync(raw.data(), d_raw_windows, raw.size() * sizeof(int2),
                                       hipMemcpyDeviceToHost, ctx->stream));
     EPSEON_HIP_TRY(hipStreamSynchronize(ctx->stream));
+    // The windows wait for nothing but the tables; the lists and the cleared
+    // scan results (16 bytes per energy) follow while the host sorts the
+    // windows out.
+    EPSEON_HIP_TRY(launch_load_lists(ctx->stream, d_runs, static_cast<int32_t>(runs.size()), d_wave_tasks, d_psi_runs,
+                                     static_cast<int32_t>(psi_runs.size()), d_all_psi_tasks, ctx->d_far,
+                                     static_cast<int64_t>(ne)));
     std::vector<BandWindow> win_full(raw.size()), win_band(raw.size());
     std::vector<TableJob> jobs_full, jobs_band;
     int64_t band_total = 0;
@@ -1345,8 +1349,8 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         up.add(band_bins, &ctx->d_xcd_bins_band);
         up.add(band_runs, &d_band_runs);
         EPSEON_HIP_TRY(up.send(a, ctx->stream));
-        EPSEON_HIP_TRY(launch_task_lists(ctx->stream, d_band_runs, static_cast<int32_t>(band_runs.size()),
-                                         ctx->d_xcd_scan_tasks_band, nullptr, 0, nullptr));
+        EPSEON_HIP_TRY(launch_load_lists(ctx->stream, d_band_runs, static_cast<int32_t>(band_runs.size()),
+                                         ctx->d_xcd_scan_tasks_band, nullptr, 0, nullptr, nullptr, 0));
     }
     ctx->h_win_full = std::move(win_full);
     ctx->h_win_band = std::move(win_band);
