@@ -134,7 +134,8 @@ struct YShot {
 // whole launch): its loads are scalar loads.
 using ConstTable = const __attribute__((address_space(4))) double*;
 
-__device__ __forceinline__ void load16(double (&buf)[16], const ConstTable p)
+template <class Table>
+__device__ __forceinline__ void load16(double (&buf)[16], const Table p)
 {
 #pragma unroll
     for (int q = 0; q < 16; ++q)
@@ -155,7 +156,7 @@ __device__ __forceinline__ void half_block(const double (&buf)[16], Body& body)
     }
 }
 
-// The last rem < 32 steps (rem wave-uniform), from the two buffers.
+// The last rem < 32 steps, from the two buffers.
 template <int Q, class Body>
 __device__ __forceinline__ void psi_tail(const double (&a)[16], const double (&b)[16], const int32_t rem, Body& body)
 {
@@ -171,17 +172,10 @@ __device__ __forceinline__ void psi_tail(const double (&a)[16], const double (&b
 // inside the current 32-step block), body.block_end(count, full) after each
 // full block of 32 and after the tail.  Two 16-value buffers, each loaded one
 // half-block ahead.  Reads up to 47 values past `steps` (tables are padded).
-template <class Body>
-__device__ __forceinline__ void psi_walk(const double* __restrict__ table, const int32_t steps, Body& body)
+template <class Table, class Body>
+__device__ __forceinline__ void psi_walk_from(Table p, const int32_t steps, Body& body)
 {
     const int32_t nsb = steps >> 5;
-    // Wave-uniform; stated, because a pointer whose parts were loaded after a
-    // store sits in vector registers, and vector loads of the table would wait
-    // in line behind the pass's own stores.
-    const uint64_t at = reinterpret_cast<uint64_t>(table);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
-    ConstTable p = (ConstTable)((static_cast<uint64_t>(hi) << 32) | lo);
     double a[16], b[16];
     load16(a, p);
     for (int32_t sb = 0; sb < nsb; ++sb) {
@@ -198,6 +192,20 @@ __device__ __forceinline__ void psi_walk(const double* __restrict__ table, const
         psi_tail<0>(a, b, rem, body);
         body.block_end(rem, false);
     }
+}
+
+// The walk of a wavefront whose lanes share the segment.
+template <class Body>
+__device__ __forceinline__ void psi_walk(const double* __restrict__ table, const int32_t steps, Body& body)
+{
+    // Wave-uniform; stated, because a pointer whose parts were loaded after a
+    // store sits in vector registers, and vector loads of the table would wait
+    // in line behind the pass's own stores.
+    const uint64_t at = reinterpret_cast<uint64_t>(table);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
+    ConstTable p = (ConstTable)((static_cast<uint64_t>(hi) << 32) | lo);
+    psi_walk_from(p, steps, body);
 }
 
 // frexp exponent of m (0 for m = 0).
@@ -407,17 +415,34 @@ __device__ __forceinline__ void psi_start(YShot& s, const PotentialRecord& P, co
 
 // Pass 1a: one wavefront per eigenfunction task (potential, 64 levels, side,
 // segment): each converged level's segment matrix and Gram sums.
+// kPacked: the wavefronts of a potential's tasks take its (segment, level)
+// pairs in order, 64 each (a pair's number is its slot), and those past the
+// last pair leave.  A lane then loads its own segment's values.
+template <bool kPacked>
 __global__ __launch_bounds__(64) void psi_segment_kernel(
     const double* __restrict__ uv, const double* __restrict__ uvr,
     const PotentialRecord* __restrict__ pots, const PsiTask* __restrict__ tasks,
     const double* __restrict__ levels, const int32_t* __restrict__ status,
     PsiSegMatrix* __restrict__ mats)
 {
-    const PsiTask task = tasks[blockIdx.x];
+    PsiTask task = tasks[blockIdx.x];
     const PotentialRecord& P = pots[task.potential];
-    const int32_t l = task.first + static_cast<int32_t>(threadIdx.x);
-    if (P.flags != 0 || l >= P.level_count)
+    int32_t l = task.first + static_cast<int32_t>(threadIdx.x);
+    if (P.flags != 0)
         return;
+    if constexpr (kPacked) {
+        const int32_t segment = (task.side == 0 ? 0 : P.psi_segs_left) + task.segment;
+        const int64_t pair =
+            (static_cast<int64_t>(segment) * ((P.level_count + 63) / 64) + task.first / 64) * 64 + threadIdx.x;
+        if (pair >= static_cast<int64_t>(P.psi_segs_left + P.psi_segs_right) * P.level_count)
+            return;
+        const int32_t at = static_cast<int32_t>(pair / P.level_count);
+        l = static_cast<int32_t>(pair - static_cast<int64_t>(at) * P.level_count);
+        task.side = at < P.psi_segs_left ? 0 : 1;
+        task.segment = at - (task.side == 0 ? 0 : P.psi_segs_left);
+    } else if (l >= P.level_count) {
+        return;
+    }
     const int64_t o = P.level_offset + l;
     if (!level_active(status, o))
         return;
@@ -434,7 +459,10 @@ __global__ __launch_bounds__(64) void psi_segment_kernel(
     B.c10 = opaque(10.0);
     B.fm = e - g.p[g.j0];
     B.f = e - g.p[g.j0 + 1];
-    psi_walk(g.p + 2 + g.j0, g.steps, B);
+    if constexpr (kPacked)
+        psi_walk_from(g.p + 2 + g.j0, g.steps, B);
+    else
+        psi_walk(g.p + 2 + g.j0, g.steps, B);
     B.renormalize();
     mats[psi_slot(P, task.side, task.segment, l)] =
         PsiSegMatrix{B.ay, B.aym, B.ad, B.by, B.bym, B.bd, B.saa, B.sab, B.sbb, B.ex, 0};
@@ -691,13 +719,17 @@ __global__ __launch_bounds__(64 * W) void level_vjp_kernel(
 // ---------------------------------------------------------------- launchers
 
 hipError_t launch_normalize(hipStream_t stream, const double* uv, const double* uvr,
-                            const PotentialRecord* pots, const PsiTask* psi_tasks, int32_t n_psi_tasks,
+                            const PotentialRecord* pots, const PsiTask* psi_tasks, int32_t n_psi_tasks, bool packed,
                             const WaveTask* tasks, int32_t n_tasks, const double* levels,
                             const int32_t* status, PsiSegMatrix* mats, PsiCheckpoint* ckpt, LevelNorm* norms)
 {
     if (n_psi_tasks > 0) {
-        hipLaunchKernelGGL(psi_segment_kernel, dim3(static_cast<unsigned>(n_psi_tasks)), dim3(64), 0, stream,
-                           uv, uvr, pots, psi_tasks, levels, status, mats);
+        if (packed)
+            hipLaunchKernelGGL(psi_segment_kernel<true>, dim3(static_cast<unsigned>(n_psi_tasks)), dim3(64), 0, stream,
+                               uv, uvr, pots, psi_tasks, levels, status, mats);
+        else
+            hipLaunchKernelGGL(psi_segment_kernel<false>, dim3(static_cast<unsigned>(n_psi_tasks)), dim3(64), 0, stream,
+                               uv, uvr, pots, psi_tasks, levels, status, mats);
         if (const hipError_t e = hipGetLastError(); e != hipSuccess)
             return e;
     }

@@ -51,7 +51,7 @@ hipError_t launch_band_windows(hipStream_t, const double*, const PotentialRecord
 hipError_t launch_level_summary(hipStream_t, const PotentialRecord*, const WaveTask*, int32_t, const int32_t*,
                                 const int32_t*, const int32_t*, int64_t*);
 hipError_t launch_normalize(hipStream_t, const double*, const double*, const PotentialRecord*,
-                            const PsiTask*, int32_t, const WaveTask*, int32_t, const double*, const int32_t*,
+                            const PsiTask*, int32_t, bool, const WaveTask*, int32_t, const double*, const int32_t*,
                             PsiSegMatrix*, PsiCheckpoint*, LevelNorm*);
 hipError_t launch_eigenfunctions(hipStream_t, const double*, const double*, const PotentialRecord*,
                                  const PsiTask*, int32_t, const double*, const int32_t*,
@@ -404,6 +404,7 @@ struct epseon_ctx {
     PsiTask* d_vjp_lists[4] = {};
     int32_t n_vjp[4] = {};
     PsiTask* d_psi_tasks = nullptr;
+    int64_t psi_pairs = 0;  // (segment, level) pairs of the eigenfunction tasks
     std::vector<int32_t> cum_psi_tasks;
     // Eigenfunction-shot checkpoints written by the normalisation pass
     // (carved from the arena on first use).
@@ -1114,9 +1115,13 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     }
     const int64_t psi_at = n_psi_tasks;
     ctx->cum_psi_tasks.assign(1, 0);
+    ctx->psi_pairs = 0;
     for (int32_t p : order) {
-        add_psi(p, (ctx->rec[static_cast<size_t>(p)].level_count + 63) / 64);
+        const PotentialRecord& r = ctx->rec[static_cast<size_t>(p)];
+        add_psi(p, (r.level_count + 63) / 64);
         ctx->cum_psi_tasks.push_back(static_cast<int32_t>(n_psi_tasks - psi_at));
+        if (usable(r))
+            ctx->psi_pairs += static_cast<int64_t>(r.psi_segs_left + r.psi_segs_right) * r.level_count;
     }
 
     const size_t np = static_cast<size_t>(std::max<int64_t>(pts, 1));
@@ -1444,6 +1449,22 @@ int32_t segmented_lanes(const epseon_ctx* ctx)
     while (lanes < 256 && ctx->total_levels * (lanes / 64) * 2 <= 2048)
         lanes *= 2;
     return lanes;
+}
+
+// Whether the normalisation's segment pass packs a potential's (segment,
+// level) pairs into full wavefronts: when that takes at least a sixteenth of
+// the wavefronts away and each SIMD has kPsiPackTasks / 1024 of them, so that
+// their number is what the pass costs.  256 x 50,000 points with 41 levels 581
+// -> 416 us; 96 x 50,000 points (normalisation, both passes): 17 levels 244 ->
+// 120 us, 48 levels 261 -> 224, 60 levels 270 -> 259, 68 levels 1,195 -> 285;
+// 41 levels on 32 x 50,000 points 112 -> 95, but on 64 x 10,000 points (5,000
+// tasks) 56 -> 58 and on 16 x 50,000 (3,100) 65 -> 67: lanes that load their
+// own values wait for vector loads.
+constexpr int64_t kPsiPackTasks = 6144;
+bool psi_packed(const epseon_ctx* ctx)
+{
+    const int64_t tasks = ctx->cum_psi_tasks.back();
+    return tasks >= kPsiPackTasks && ctx->psi_pairs <= 60 * tasks;
 }
 
 // Levels per segmented block: in 64-lane blocks four (each table load then
@@ -2150,7 +2171,7 @@ int epseon_normalize(epseon_ctx* ctx)
     }
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[4], ctx->stream));
     EPSEON_HIP_TRY(launch_normalize(ctx->stream, ctx->d_uv, ctx->d_uvr, ctx->d_rec, ctx->d_psi_tasks,
-                                    ctx->cum_psi_tasks.back(), ctx->d_refine_tasks, ctx->n_refine_tasks,
+                                    ctx->cum_psi_tasks.back(), psi_packed(ctx), ctx->d_refine_tasks, ctx->n_refine_tasks,
                                     ctx->d_levels, ctx->d_status, ctx->d_psi_mats, ctx->d_ckpt,
                                     ctx->d_norms));
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[5], ctx->stream));
@@ -2310,7 +2331,7 @@ int epseon_level_vjp_noalloc(epseon_ctx* ctx, const double* grad_levels_device, 
     // The context's own checkpoints (epseon_normalize) are left as they are.
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[6], ctx->stream));
     EPSEON_HIP_TRY(launch_normalize(ctx->stream, ctx->d_uv, ctx->d_uvr, ctx->d_rec, ctx->d_psi_tasks,
-                                    ctx->cum_psi_tasks.back(), ctx->d_refine_tasks, ctx->n_refine_tasks,
+                                    ctx->cum_psi_tasks.back(), psi_packed(ctx), ctx->d_refine_tasks, ctx->n_refine_tasks,
                                     ctx->d_levels, ctx->d_status, mats, ckpt, ctx->d_norms));
     const hipStream_t streams[4] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
