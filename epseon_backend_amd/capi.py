@@ -207,6 +207,15 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "epseon_level_vjp_noalloc": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "epseon_get_all_wavefunctions": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32]),
     "epseon_get_eigenfunction_size": (ctypes.c_int, [ctypes.c_void_p, _c_int64_p]),
+    "epseon_morse_chunks": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64]),
+    "epseon_morse_table": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 4 + [ctypes.c_int64] * 2 + [ctypes.c_void_p] * 3,
+    ),
+    "epseon_morse_vjp": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 4 + [ctypes.c_int64] * 2 + [ctypes.c_void_p] * 3,
+    ),
 }
 
 _LIB: ctypes.CDLL | None = None

@@ -404,6 +404,26 @@ int epseon_get_sizes(epseon_ctx* ctx, int32_t* potentials, int64_t* points, int6
 /* Counters and device times of the last phases. */
 int epseon_get_stats(epseon_ctx* ctx, epseon_stats* stats);
 
+/* ---- Morse tables ------------------------------------------------------- */
+
+/* Workgroups per potential of the two calls below, 0 for sizes they refuse
+ * (none, or more than one launch takes). */
+int epseon_morse_chunks(int64_t rows, int64_t points);
+
+/* V = D (1 - exp(-a (r - r_e)))^2 of each of `rows` potentials (r, v: rows of
+ * `points` doubles one after the other; de, a, re: one per row) and, where d
+ * is not NULL, d = r - r_e.  Device pointers of the current device; enqueued
+ * on `stream` (a hipStream_t), nothing is allocated or waited for. */
+int epseon_morse_table(const double* r, const double* de, const double* a, const double* re, int64_t rows,
+                       int64_t points, double* v, double* d, void* stream);
+
+/* Gradients of a loss with respect to D, a and r_e (grad: 3 x rows) from its
+ * gradient g with respect to V and the forward call's d.  part: 3 x rows x
+ * epseon_morse_chunks doubles of scratch, unused with one chunk.  The sums'
+ * order depends on `points` alone.  As above otherwise. */
+int epseon_morse_vjp(const double* g, const double* d, const double* de, const double* a, int64_t rows,
+                     int64_t points, double* part, double* grad, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
