@@ -190,6 +190,14 @@ constexpr int64_t kDeviceStatsMinPoints = 100000;
 constexpr int64_t kSpreadMaxScanWavesPerSimd = 48;
 constexpr double kSpreadMinSteps = 4096.0;
 
+// Tasks at the end of a windowed scan's bins that are ordered longest first
+// across potentials: four times what an XCD holds at two wavefronts per SIMD.
+// From kSpreadMinSteps on average (scans, before and after): 256 x 50,000
+// points 2.55 -> 2.10 ms, 512 x 20,000 1.94 -> 1.80, 1,024 x 8,000 0.44 ->
+// 0.32, 256 ragged potentials 0.81 -> 0.69, 512 1.48 -> 1.45, 4,096 unchanged;
+// shorter ones (1,024 x 2,000: 0.13 ms) have no tail worth the ordering.
+constexpr int32_t kTailTasks = 1024;
+
 // Automatic windows need at least this many scan wavefronts per SIMD.
 constexpr int64_t kWindowsMinScanWavesPerSimd = 8;
 
@@ -1285,52 +1293,88 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         if (ctx->wide_lanes == 0)
             jobs_wide.clear();
     }
-    // Windowed scan: a task's work is its trial energies times its band
-    // window's steps.  Its own XCD bins, and within each chunk the longest
-    // tasks first: runs of equal work (a band's groups, the partly filled last
-    // group) by decreasing work.
-    std::vector<double> band_task_work(static_cast<size_t>(ctx->n_scan_tasks));
+    // Windowed scan: a task's work is its band window's steps (a partly filled
+    // wavefront takes as long as a full one).  Its own XCD bins, and within
+    // each chunk the longest tasks first, in runs of equal work (a band's
+    // groups).  The last kTailTasks of a bin are ordered longest first across
+    // their chunks (to 1/64 of the longest): in order of the chunks a batch of
+    // equal grids ends with whole shots that start when most SIMDs have run dry.
+    std::vector<int32_t> band_task_work(static_cast<size_t>(ctx->n_scan_tasks));
+    double wave_steps = 0.0;
     for (size_t k = 0; k < static_cast<size_t>(count); ++k) {
         const PotentialRecord& r = rec_at(k);
         const BandWindow* w = &win_band[static_cast<size_t>(order[k]) * kBands];
         int32_t band = 0;
         for (int32_t t = ctx->cum_scan_tasks[k], j = 0; t < ctx->cum_scan_tasks[k + 1]; ++t, j += 64) {
             band = host_group_band(r, j, band);
-            const double x = static_cast<double>(std::min(64, r.n_energies - j)) *
-                             static_cast<double>(w[band].hi - w[band].lo - 1);
-            band_task_work[static_cast<size_t>(t)] = x;
-            scan_pu_band += x;
+            const int32_t n = w[band].hi - w[band].lo - 1;
+            band_task_work[static_cast<size_t>(t)] = n;
+            wave_steps += n;
+            scan_pu_band += static_cast<double>(std::min(64, r.n_energies - j)) * static_cast<double>(n);
         }
     }
     std::vector<int32_t> band_bins;
     std::vector<TaskRun> band_runs;
     {
         struct Run {
-            int32_t i0, i1;
-            double work;
+            int32_t k, i0, i1, work;
         };
-        std::vector<Run> of_chunk;
+        constexpr int32_t kBuckets = 64;
+        std::vector<Run> runs_of, sorted;
         int64_t at = 0;
+        const auto emit = [&](const Run& q) {
+            band_runs.push_back({at, order[static_cast<size_t>(q.k)], 64 * q.i0, 64, q.i1 - q.i0});
+            at += q.i1 - q.i0;
+        };
+        const auto add_runs = [&](const TaskChunk& c) {
+            const int32_t* tw = &band_task_work[static_cast<size_t>(ctx->cum_scan_tasks[static_cast<size_t>(c.k)])];
+            for (int32_t i = c.i0; i < c.i1; ++i) {
+                if (i == c.i0 || runs_of.back().work != tw[i])
+                    runs_of.push_back({c.k, i, i, tw[i]});
+                runs_of.back().i1 = i + 1;
+            }
+        };
         const auto work = [&](size_t k, int32_t i0, int32_t i1) {
             double sum = 0.0;
             for (int32_t i = i0; i < i1; ++i)
                 sum += band_task_work[static_cast<size_t>(ctx->cum_scan_tasks[k] + i)];
             return sum;
         };
-        for (const TaskChunk& c : xcd_chunks(ctx->cum_scan_tasks, work, band_bins, ctx->xcd_max_bin_band)) {
-            const double* tw = &band_task_work[static_cast<size_t>(ctx->cum_scan_tasks[static_cast<size_t>(c.k)])];
-            of_chunk.clear();
-            for (int32_t i = c.i0; i < c.i1; ++i) {
-                if (of_chunk.empty() || of_chunk.back().work != tw[i])
-                    of_chunk.push_back({i, i, tw[i]});
-                of_chunk.back().i1 = i + 1;
+        const std::vector<TaskChunk> chunks =
+            xcd_chunks(ctx->cum_scan_tasks, work, band_bins, ctx->xcd_max_bin_band);
+        const int32_t tail = wave_steps >= kSpreadMinSteps * ctx->n_scan_tasks ? kTailTasks : 0;
+        size_t c = 0;
+        for (size_t x = 0; x < 8; ++x) {
+            const int32_t end = band_bins[x + 1];
+            while (c < chunks.size() && at < end && end - at > tail) {
+                runs_of.clear();
+                add_runs(chunks[c++]);
+                std::stable_sort(runs_of.begin(), runs_of.end(),
+                                 [](const Run& p, const Run& q) { return p.work > q.work; });
+                for (const Run& q : runs_of)
+                    emit(q);
             }
-            std::stable_sort(of_chunk.begin(), of_chunk.end(),
-                             [](const Run& x, const Run& y) { return x.work > y.work; });
-            for (const Run& q : of_chunk) {
-                band_runs.push_back({at, order[static_cast<size_t>(c.k)], 64 * q.i0, 64, q.i1 - q.i0});
-                at += q.i1 - q.i0;
+            runs_of.clear();
+            int32_t longest_run = 1;
+            for (int64_t t = at; t < end; ++c) {
+                add_runs(chunks[c]);
+                t += chunks[c].i1 - chunks[c].i0;
             }
+            for (const Run& q : runs_of)
+                longest_run = std::max(longest_run, q.work);
+            const auto bucket = [&](const Run& q) {
+                return static_cast<size_t>(kBuckets - 1 - static_cast<int64_t>(q.work) * (kBuckets - 1) / longest_run);
+            };
+            size_t first[kBuckets + 1] = {};
+            for (const Run& q : runs_of)
+                ++first[bucket(q) + 1];
+            for (size_t i = 1; i <= kBuckets; ++i)
+                first[i] += first[i - 1];
+            sorted.resize(runs_of.size());
+            for (const Run& q : runs_of)
+                sorted[first[bucket(q)]++] = q;
+            for (const Run& q : sorted)
+                emit(q);
         }
     }
     EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max(ctx->n_scan_tasks, 1)), &ctx->d_xcd_scan_tasks_band));
