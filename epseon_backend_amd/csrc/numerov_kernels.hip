@@ -2256,8 +2256,14 @@ __device__ __forceinline__ void tables_in_lanes(SegControl<K>& ctl, const int32_
 // walk, three padded with a copy of the first), each grid value loaded once
 // for all of them; counted shots and levels of other windows shoot apart.
 // Every level's arithmetic is that of a block of its own.
+//
+// Registers: blocks of 128 and 256 lanes are for batches of at most 2,048
+// wavefronts, two per SIMD, so they take the registers of two (231, against
+// 168 and 64 to 96 bytes of scratch per lane for three): 12 potentials of
+// 10,007 points 40.3 -> 38.1 us, 32 of 8,000 60.2 -> 55.9, one light molecule
+// 31.0 -> 29.1, one table of 1,000,000 points 339 -> 342.
 template <int T, bool TABLE, int K>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(K == 4 ? 2 : 3))) void
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(K == 4 || T > 64 ? 2 : 3))) void
 numerov_refine_segmented_kernel(const double* __restrict__ uv, const double* __restrict__ segtab,
                                 const PotentialRecord* __restrict__ pots, const BandWindow* __restrict__ windows,
                                 const WaveTask* __restrict__ tasks, const int32_t n_tasks,
