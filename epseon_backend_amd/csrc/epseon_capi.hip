@@ -408,9 +408,9 @@ struct epseon_ctx {
     double* d_grad_levels = nullptr;
     // Adjoint tasks (potential, side, segment) grouped by block width (1..4
     // wavefronts), and the eigenfunction tasks (potential, 64 levels, side,
-    // segment) in potential task order with cumulative counts.
+    // segment), each in potential task order with cumulative counts.
     PsiTask* d_vjp_lists[4] = {};
-    int32_t n_vjp[4] = {};
+    std::vector<int32_t> cum_vjp[4];
     PsiTask* d_psi_tasks = nullptr;
     int64_t psi_pairs = 0;  // (segment, level) pairs of the eigenfunction tasks
     std::vector<int32_t> cum_psi_tasks;
@@ -418,7 +418,9 @@ struct epseon_ctx {
     // (carved from the arena on first use).
     PsiCheckpoint* d_ckpt = nullptr;
     PsiSegMatrix* d_psi_mats = nullptr;
-    int64_t ckpt_total = 0;
+    int64_t ckpt_total = 0;  // (segment, level) pairs, cumulative in task order, and with long segments
+    std::vector<int64_t> cum_ckpt;
+    int64_t ckpt_long = 0;
     // Scratch for host-side outputs, carved from the arena on first use.
     double* d_stage = nullptr;
     size_t stage_elems = 0;
@@ -903,7 +905,7 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         EPSEON_HIP_TRY(hipStreamSynchronize(ctx->stream));
     }
 
-    int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0, psi_waves = 0;
+    int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0, ckpt_long = 0;
     int32_t max_seg_rows = 0, longest = 0;
     double scan_pu = 0.0;
     for (int32_t p = 0; p < count; ++p) {
@@ -961,11 +963,15 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         max_seg_rows = std::max(max_seg_rows, seg_rows(r.n_points, r.flags, r.level_count));
         if (seg_total > INT32_MAX)
             return fail(EPSEON_ERR_INVALID, "batch too large for the segment table");
-        r.psi_seg_len = psi_seg_len(r.n_points);
-        if (r.flags == EPSEON_POT_OK)
-            psi_waves += static_cast<int64_t>((d.level_count + 63) / 64) *
-                         ((r.match + r.psi_seg_len - 1) / r.psi_seg_len +
-                          (r.n_points - 2 - r.match + r.psi_seg_len - 1) / r.psi_seg_len);
+        r.psi_seg_len = psi_seg_len(r.n_points, r.level_count);
+        const auto segments = [&](int32_t steps, int32_t len) { return (steps + len - 1) / len; };
+        r.psi_segs_left = segments(r.match, r.psi_seg_len);
+        r.psi_segs_right = segments(r.n_points - 2 - r.match, r.psi_seg_len);
+        if (r.flags == EPSEON_POT_OK) {
+            const int32_t len = psi_long_seg_len(r.n_points);
+            ckpt_long += static_cast<int64_t>(d.level_count) *
+                         (segments(r.match, len) + segments(r.n_points - 2 - r.match, len));
+        }
         r.chunk0 = table_chunk0[static_cast<size_t>(p)];
         r.user_offset = v_offsets[p];
         r.psi_offset = psi_total;
@@ -982,25 +988,12 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         if (r.flags == EPSEON_POT_OK)
             scan_pu += static_cast<double>(r.n_points - 2) * static_cast<double>(d.n_energies);
     }
-    // Eigenfunction shots run in segments of psi_seg_len steps; the
-    // normalisation pass leaves a checkpoint per level at each segment start
-    // (slot 0 of each side is unused).
-    for (PotentialRecord& r : ctx->rec) {
-        if (psi_waves < kPsiFewWaves)
-            r.psi_seg_len = psi_short_seg_len(r.n_points);
-        r.psi_segs_left = (r.match + r.psi_seg_len - 1) / r.psi_seg_len;
-        r.psi_segs_right = (r.n_points - 2 - r.match + r.psi_seg_len - 1) / r.psi_seg_len;
-        r.psi_ckpt = ckpt_total;
-        if (r.flags == EPSEON_POT_OK)
-            ckpt_total += static_cast<int64_t>(r.level_count) * (r.psi_segs_left + r.psi_segs_right);
-    }
     ctx->total_points = pts;
     ctx->total_energies = en;
     ctx->total_levels = lv;
     ctx->scan_pu_full = scan_pu;
     ctx->user_span = user_span;
     ctx->psi_total = psi_total;
-    ctx->ckpt_total = ckpt_total;
 
     // Work lists: one wavefront per 64 trial energies (scan) or 64 levels
     // (refine), longest grids first so the dispatcher drains large items early.
@@ -1012,6 +1005,19 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     ctx->order_pos.assign(static_cast<size_t>(count), 0);
     for (int32_t k = 0; k < count; ++k)
         ctx->order_pos[static_cast<size_t>(order[static_cast<size_t>(k)])] = k;
+    // Eigenfunction shots run in segments of psi_seg_len steps; the
+    // normalisation pass keeps a map and a checkpoint per (segment, level)
+    // pair, in task order.
+    ctx->cum_ckpt.assign(1, 0);
+    for (int32_t p : order) {
+        PotentialRecord& r = ctx->rec[static_cast<size_t>(p)];
+        r.psi_ckpt = ckpt_total;
+        if (r.flags == EPSEON_POT_OK)
+            ckpt_total += static_cast<int64_t>(r.level_count) * (r.psi_segs_left + r.psi_segs_right);
+        ctx->cum_ckpt.push_back(ckpt_total);
+    }
+    ctx->ckpt_total = ckpt_total;
+    ctx->ckpt_long = ckpt_long;
     // The lists themselves are written on the device from runs of consecutive
     // tasks, one run per potential and list or per chunk of a binned list.
     std::vector<TaskRun> runs;
@@ -1116,10 +1122,12 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     int64_t vjp_at[4];
     for (int32_t w = 0; w < 4; ++w) {
         vjp_at[w] = n_psi_tasks;
-        for (int32_t p : order)
+        ctx->cum_vjp[w].assign(1, 0);
+        for (int32_t p : order) {
             if (std::clamp((ctx->rec[static_cast<size_t>(p)].level_count + 63) / 64, 1, 4) == w + 1)
                 add_psi(p, 1);
-        ctx->n_vjp[w] = static_cast<int32_t>(n_psi_tasks - vjp_at[w]);
+            ctx->cum_vjp[w].push_back(static_cast<int32_t>(n_psi_tasks - vjp_at[w]));
+        }
     }
     const int64_t psi_at = n_psi_tasks;
     ctx->cum_psi_tasks.assign(1, 0);
@@ -2254,6 +2262,28 @@ int write_wavefunctions(epseon_ctx* ctx, size_t k0, size_t k1, int64_t base, siz
     return EPSEON_OK;
 }
 
+// Adjoint of the potentials [k0, k1) in task order from their checkpoints.  The
+// four block-width classes touch disjoint potentials: one stream each, joined.
+hipError_t run_level_vjp(epseon_ctx* ctx, size_t k0, size_t k1, const PsiCheckpoint* ckpt, const double* grad_levels,
+                         double* grad_v)
+{
+    const hipStream_t streams[4] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
+    hipError_t e = hipEventRecord(ctx->ev_fork, ctx->stream);
+    for (int w = 1; w < 4 && e == hipSuccess; ++w)
+        e = hipStreamWaitEvent(streams[w], ctx->ev_fork, 0);
+    for (int w = 0; w < 4 && e == hipSuccess; ++w) {
+        const int32_t t0 = ctx->cum_vjp[w][k0], t1 = ctx->cum_vjp[w][k1];
+        e = launch_level_vjp(streams[w], w + 1, ctx->d_uv, ctx->d_uvr, ctx->d_rec, ctx->d_vjp_lists[w] + t0, t1 - t0,
+                             ctx->d_levels, ctx->d_status, ctx->d_norms, ckpt, grad_levels, grad_v);
+    }
+    for (int w = 1; w < 4 && e == hipSuccess; ++w) {
+        e = hipEventRecord(ctx->ev_join_aux[w - 1], streams[w]);
+        if (e == hipSuccess)
+            e = hipStreamWaitEvent(ctx->stream, ctx->ev_join_aux[w - 1], 0);
+    }
+    return e;
+}
+
 }  // namespace
 
 int epseon_get_wavefunctions(epseon_ctx* ctx, int32_t potential, double* psi, int32_t mem)
@@ -2314,19 +2344,7 @@ int epseon_level_vjp(epseon_ctx* ctx, const double* grad_levels, double* grad_v,
         out = ctx->d_stage;
     }
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[6], ctx->stream));
-    // The four block-width classes touch disjoint potentials: one stream each.
-    const hipStream_t streams[4] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
-    EPSEON_HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
-    for (int w = 1; w < 4; ++w)
-        EPSEON_HIP_TRY(hipStreamWaitEvent(streams[w], ctx->ev_fork, 0));
-    for (int w = 0; w < 4; ++w)
-        EPSEON_HIP_TRY(launch_level_vjp(streams[w], w + 1, ctx->d_uv, ctx->d_uvr, ctx->d_rec,
-                                        ctx->d_vjp_lists[w], ctx->n_vjp[w], ctx->d_levels,
-                                        ctx->d_status, ctx->d_norms, ctx->d_ckpt, g, out));
-    for (int w = 1; w < 4; ++w) {
-        EPSEON_HIP_TRY(hipEventRecord(ctx->ev_join_aux[w - 1], streams[w]));
-        EPSEON_HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->ev_join_aux[w - 1], 0));
-    }
+    EPSEON_HIP_TRY(run_level_vjp(ctx, 0, n_potentials(ctx), ctx->d_ckpt, g, out));
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[7], ctx->stream));
     ctx->vjp_timed = true;
     if (mem == EPSEON_MEM_HOST) {
@@ -2353,41 +2371,47 @@ int epseon_level_vjp_noalloc(epseon_ctx* ctx, const double* grad_levels_device, 
     if (grad_v_device == nullptr || (grad_levels_device == nullptr && ctx->total_levels > 0))
         return fail(EPSEON_ERR_INVALID, "null gradient pointer");
     // Segment maps and checkpoints of the normalisation pass, both carved
-    // from the device's scratch array.
-    const size_t slots = static_cast<size_t>(std::max<int64_t>(ctx->ckpt_total, 1));
-    const size_t ckpt_bytes = (slots * sizeof(PsiCheckpoint) + 255) & ~size_t(255);
-    const size_t need = ckpt_bytes + slots * sizeof(PsiSegMatrix);
-    if (need > kNoAllocScratchBytes) {
+    // from the device's scratch array.  The maximum counts long segments.
+    const auto bytes = [](int64_t pairs) {
+        return ((static_cast<size_t>(pairs) * sizeof(PsiCheckpoint) + 255) & ~size_t(255)) +
+               static_cast<size_t>(pairs) * sizeof(PsiSegMatrix);
+    };
+    const int64_t pairs = std::max<int64_t>(ctx->ckpt_long, 1);
+    if (bytes(pairs) > kNoAllocScratchBytes) {
         char msg[256];
         std::snprintf(msg, sizeof msg,
-                      "epseon_level_vjp_noalloc: the batch needs %zu bytes of scratch (%zu eigenfunction-shot "
+                      "epseon_level_vjp_noalloc: the batch needs %zu bytes of scratch (%lld eigenfunction-shot "
                       "segments), above the %zu-byte maximum",
-                      need, slots, kNoAllocScratchBytes);
+                      bytes(pairs), static_cast<long long>(pairs), kNoAllocScratchBytes);
         return fail(EPSEON_ERR_INVALID, msg);
     }
     void* base = scratch_of(ctx->device);
     if (base == nullptr)
         return fail(EPSEON_ERR_DEVICE, "epseon_level_vjp_noalloc: no scratch on this device");
-    PsiCheckpoint* ckpt = static_cast<PsiCheckpoint*>(base);
-    PsiSegMatrix* mats = reinterpret_cast<PsiSegMatrix*>(static_cast<char*>(base) + ckpt_bytes);
     // The scratch holds whatever the last call on this device left, so the
     // normalisation always runs; every slot a kernel reads is written first.
     // The context's own checkpoints (epseon_normalize) are left as they are.
+    // Potentials go in task order, as many at a time as the scratch holds the
+    // (shorter) segments of: one always fits.
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[6], ctx->stream));
-    EPSEON_HIP_TRY(launch_normalize(ctx->stream, ctx->d_uv, ctx->d_uvr, ctx->d_rec, ctx->d_psi_tasks,
-                                    ctx->cum_psi_tasks.back(), psi_packed(ctx), ctx->d_refine_tasks, ctx->n_refine_tasks,
-                                    ctx->d_levels, ctx->d_status, mats, ckpt, ctx->d_norms));
-    const hipStream_t streams[4] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
-    EPSEON_HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
-    for (int w = 1; w < 4; ++w)
-        EPSEON_HIP_TRY(hipStreamWaitEvent(streams[w], ctx->ev_fork, 0));
-    for (int w = 0; w < 4; ++w)
-        EPSEON_HIP_TRY(launch_level_vjp(streams[w], w + 1, ctx->d_uv, ctx->d_uvr, ctx->d_rec,
-                                        ctx->d_vjp_lists[w], ctx->n_vjp[w], ctx->d_levels, ctx->d_status,
-                                        ctx->d_norms, ckpt, grad_levels_device, grad_v_device));
-    for (int w = 1; w < 4; ++w) {
-        EPSEON_HIP_TRY(hipEventRecord(ctx->ev_join_aux[w - 1], streams[w]));
-        EPSEON_HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->ev_join_aux[w - 1], 0));
+    const size_t np = n_potentials(ctx);
+    for (size_t k0 = 0, k1 = 0; k0 < np; k0 = k1) {
+        const int64_t at = ctx->cum_ckpt[k0];
+        while (k1 < np && bytes(ctx->cum_ckpt[k1 + 1] - at) <= kNoAllocScratchBytes)
+            ++k1;
+        if (k1 == k0)
+            return fail(EPSEON_ERR_DEVICE, "epseon_level_vjp_noalloc: one potential exceeds the scratch");
+        // Slots are numbered over the whole batch.
+        const int64_t slots = ctx->cum_ckpt[k1] - at;
+        const size_t ckpt_bytes = bytes(slots) - static_cast<size_t>(slots) * sizeof(PsiSegMatrix);
+        PsiCheckpoint* ckpt = static_cast<PsiCheckpoint*>(base) - at;
+        PsiSegMatrix* mats = reinterpret_cast<PsiSegMatrix*>(static_cast<char*>(base) + ckpt_bytes) - at;
+        const int32_t p0 = ctx->cum_psi_tasks[k0], p1 = ctx->cum_psi_tasks[k1];
+        const int32_t r0 = ctx->cum_refine_tasks[k0], r1 = ctx->cum_refine_tasks[k1];
+        EPSEON_HIP_TRY(launch_normalize(ctx->stream, ctx->d_uv, ctx->d_uvr, ctx->d_rec, ctx->d_psi_tasks + p0, p1 - p0,
+                                        psi_packed(ctx), ctx->d_refine_tasks + r0, r1 - r0, ctx->d_levels,
+                                        ctx->d_status, mats, ckpt, ctx->d_norms));
+        EPSEON_HIP_TRY(run_level_vjp(ctx, k0, k1, ckpt, grad_levels_device, grad_v_device));
     }
     EPSEON_HIP_TRY(hipEventRecord(ctx->ev[7], ctx->stream));
     ctx->vjp_timed = true;

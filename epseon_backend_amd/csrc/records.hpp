@@ -117,31 +117,42 @@ constexpr int32_t seg_rows(const int32_t n_points, const int32_t flags, const in
     return ((q + segs - 1) / segs + 35) & ~1;
 }
 
-// Segment length of the eigenfunction shots of a potential with n points: a
-// multiple of 32 (the rescale block), at least 512 steps, and long enough
-// that the n - 2 steps make at most about 256 segments.
-constexpr int32_t psi_seg_len(const int32_t n_points)
+// Steps per segment that the scratch of epseon_level_vjp_noalloc is counted in
+// for a potential with n points: a multiple of 32, at least 512, and long
+// enough that the n - 2 steps make at most about 256 segments.
+constexpr int32_t psi_long_seg_len(const int32_t n_points)
 {
     const int32_t q = n_points - 2;
     const int32_t blocks = (q + 32 * 256 - 1) / (32 * 256);
     return 32 * (blocks < 16 ? 16 : blocks);
 }
 
-// Batches whose segments at that length give fewer wavefronts than this (one
-// per SIMD) leave the chip idle while each pass walks a whole segment; their
-// segments are shortened.  The walk costs about 0.08 us per step (both passes)
-// and the normalisation's chain 0.14 us per segment of a side, so the sum is
-// least near 1.3 sqrt(n) steps: a multiple of 32, at least 64 and at most
-// psi_seg_len.
-constexpr int64_t kPsiFewWaves = 1024;
-constexpr int32_t psi_short_seg_len(const int32_t n_points)
+// A potential whose (segment, level) pairs exceed this takes the long
+// segments, so that what an accepted epseon_level_vjp_noalloc call needs for
+// one potential always fits its scratch (about 18 MB of the 64 MiB).
+constexpr int64_t kPsiMaxShortPairs = 160000;
+
+// Segment length of the eigenfunction shots of a potential: a multiple of 32
+// (the rescale block).  Segment starts set how the shots round, so the length
+// depends on the potential alone and its eigenfunctions and gradients have the
+// same bits in every batch.  With few wavefronts the passes walk a whole
+// segment (about 0.08 us per step, both passes) and the normalisation's chain
+// takes 0.14 us per segment of a side: the sum is least near 1.3 sqrt(n)
+// steps.  With many, the length hardly matters (normalisation and adjoint with
+// 512 steps and with these, us: 256 x 50,000 points x 41 levels 456 + 594 and
+// 466 + 594, 256 x 7,000 x 20 128 + 131 and 66 + 118, 1,024 ragged x 24
+// 408 + 782 and 418 + 800), but below 128 steps the segments' maps become
+// the traffic (1,024 x 2,000 x 85: normalisation 259 with 64 steps, 209 with
+// 128, 200 with 512).
+constexpr int32_t psi_seg_len(const int32_t n_points, const int64_t level_count)
 {
     // 32 b >= 1.3 sqrt(n): b^2 >= 1.69 n / 1024.
-    int32_t b = 2;
+    int32_t b = 4;
     while (static_cast<int64_t>(b) * b * 1024 * 100 < static_cast<int64_t>(169) * n_points)
         ++b;
-    const int32_t most = psi_seg_len(n_points);
-    return 32 * b < most ? 32 * b : most;
+    const int32_t most = psi_long_seg_len(n_points);
+    const bool fits = level_count * (n_points / (32 * b) + 2) <= kPsiMaxShortPairs;
+    return fits && 32 * b < most ? 32 * b : most;
 }
 
 // The segments of a side's shot (side 0: from the left wall, points

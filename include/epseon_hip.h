@@ -354,11 +354,11 @@ int epseon_level_vjp(epseon_ctx* ctx, const double* grad_levels, double* grad_v,
 /* epseon_level_vjp for device pointers that allocates nothing: no hipMalloc,
  * hipFree or other allocating call, on the device or the host.  The
  * normalisation pass's segment maps and shot checkpoints (80 + 32 bytes per
- * eigenfunction-shot segment of every level, segments from
- * epseon_potential_info point counts) live in a library-owned device array of
- * EPSEON_NOALLOC_SCRATCH_BYTES per device, held until the process ends;
- * batches that need more are rejected with EPSEON_ERR_INVALID.  The
- * normalisation always runs (the array keeps the last call's contents), the
+ * shot segment of every level) live in a library-owned device array of
+ * EPSEON_NOALLOC_SCRATCH_BYTES per device, held until the process ends, as
+ * many potentials at a time as fit it.  Batches that would need more with
+ * segments of 512 steps (above 2^17 points, a 256th of the grid) are rejected
+ * with EPSEON_ERR_INVALID.  The normalisation always runs (the array keeps the last call's contents), the
  * context's own eigenfunction state is left as it was, and the result equals
  * epseon_level_vjp(ctx, grad_levels_device, grad_v_device, EPSEON_MEM_DEVICE)
  * bit for bit.  Every call on a device shares that device's array: calls
