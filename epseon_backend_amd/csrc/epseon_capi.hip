@@ -38,7 +38,7 @@ hipError_t launch_brackets(hipStream_t, const PotentialRecord*, const BandWindow
 hipError_t launch_refine(hipStream_t, int32_t, const double*, const PotentialRecord*, const BandWindow*,
                          const WaveTask*, int32_t, int32_t, const Bracket*, RefinePoints*, double, int32_t,
                          double*, int32_t*, int32_t*, int32_t*);
-hipError_t launch_refine_segmented(hipStream_t, int32_t, int32_t, const double*, const double*,
+hipError_t launch_refine_segmented(hipStream_t, int32_t, int32_t, int32_t, const double*, const double*,
                                    const PotentialRecord*, const BandWindow*, const WaveTask*, int32_t,
                                    const int32_t*, int32_t, const Bracket*, RefinePoints*, double, int32_t,
                                    double*, int32_t*, int32_t*, int32_t*);
@@ -1665,28 +1665,28 @@ hipError_t run_refine(epseon_ctx* ctx, hipStream_t stream, hipStream_t stream_b,
     else if (lanes == ctx->wide_lanes && ctx->scan_windows == ctx->wide_band)
         tab = ctx->d_segtab_wide;
     const bool whole = ctx->xcd_scan && k0 == 0 && k1 == ctx->cum_level_tasks.size() - 1;
-    const int32_t lpb = segmented_levels(ctx, lanes);
+    const int32_t lpb = segmented_levels(ctx, lanes), simds = 4 * ctx->compute_units;
     ctx->last_refine_levels = lpb;
     if (lpb == 2 || lpb == 4) {
         const int32_t g = lpb == 2 ? 0 : 1;
         const int32_t p0 = ctx->cum_group_tasks[g][k0];
         const int32_t p1 = ctx->cum_group_tasks[g][k1];
         if (whole)
-            return launch_refine_segmented(stream, lanes, lpb, ctx->d_uv, tab, ctx->d_rec, win,
+            return launch_refine_segmented(stream, simds, lanes, lpb, ctx->d_uv, tab, ctx->d_rec, win,
                                            ctx->d_xcd_group_tasks[g], p1 - p0, ctx->d_xcd_group_bins[g],
                                            ctx->xcd_max_group_bin[g], ctx->d_brackets, ctx->d_points, rel_tol,
                                            max_iter, ctx->d_levels, ctx->d_status, ctx->d_iters, ctx->d_steps);
-        return launch_refine_segmented(stream, lanes, lpb, ctx->d_uv, tab, ctx->d_rec, win,
+        return launch_refine_segmented(stream, simds, lanes, lpb, ctx->d_uv, tab, ctx->d_rec, win,
                                        ctx->d_group_tasks[g] + p0, p1 - p0, nullptr, 0, ctx->d_brackets,
                                        ctx->d_points, rel_tol, max_iter, ctx->d_levels, ctx->d_status, ctx->d_iters,
                                        ctx->d_steps);
     }
     if (whole)
-        return launch_refine_segmented(stream, lanes, 1, ctx->d_uv, tab, ctx->d_rec, win, ctx->d_xcd_level_tasks,
+        return launch_refine_segmented(stream, simds, lanes, 1, ctx->d_uv, tab, ctx->d_rec, win, ctx->d_xcd_level_tasks,
                                        t1 - t0, ctx->d_xcd_level_bins, ctx->xcd_max_level_bin, ctx->d_brackets,
                                        ctx->d_points, rel_tol, max_iter, ctx->d_levels, ctx->d_status, ctx->d_iters,
                                        ctx->d_steps);
-    return launch_refine_segmented(stream, lanes, 1, ctx->d_uv, tab, ctx->d_rec, win, ctx->d_level_tasks + t0,
+    return launch_refine_segmented(stream, simds, lanes, 1, ctx->d_uv, tab, ctx->d_rec, win, ctx->d_level_tasks + t0,
                                    t1 - t0, nullptr, 0, ctx->d_brackets, ctx->d_points, rel_tol, max_iter,
                                    ctx->d_levels, ctx->d_status, ctx->d_iters, ctx->d_steps);
 }

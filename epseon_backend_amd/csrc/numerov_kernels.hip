@@ -2257,13 +2257,16 @@ __device__ __forceinline__ void tables_in_lanes(SegControl<K>& ctl, const int32_
 // for all of them; counted shots and levels of other windows shoot apart.
 // Every level's arithmetic is that of a block of its own.
 //
-// Registers: blocks of 128 and 256 lanes are for batches of at most 2,048
-// wavefronts, two per SIMD, so they take the registers of two (231, against
-// 168 and 64 to 96 bytes of scratch per lane for three): 12 potentials of
-// 10,007 points 40.3 -> 38.1 us, 32 of 8,000 60.2 -> 55.9, one light molecule
-// 31.0 -> 29.1, one table of 1,000,000 points 339 -> 342.
-template <int T, bool TABLE, int K>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(K == 4 || T > 64 ? 2 : 3))) void
+// Registers (kWaves wavefronts per SIMD): launches of blocks of 128 and 256 lanes
+// that give each SIMD at most two wavefronts take the registers of two (231,
+// against 168 and 64 to 96 bytes of scratch per lane for three): 12 potentials
+// of 10,007 points 40.3 -> 38.1 us, 32 of 8,000 60.2 -> 55.9, one light
+// molecule 31.0 -> 29.1, one table of 1,000,000 points 339 -> 342.  Larger
+// ones, which only a fixed block width makes, need the third wavefront:
+// 87,373 levels of 1,024 x 2,000 points 3.15 -> 2.49 ms in 128 lanes and 5.85
+// -> 4.48 in 256, 64 x 20,000 x 41 levels 122 -> 113 and 161 -> 136 us.
+template <int T, bool TABLE, int K, int kWaves>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(kWaves))) void
 numerov_refine_segmented_kernel(const double* __restrict__ uv, const double* __restrict__ segtab,
                                 const PotentialRecord* __restrict__ pots, const BandWindow* __restrict__ windows,
                                 const WaveTask* __restrict__ tasks, const int32_t n_tasks,
@@ -2681,7 +2684,9 @@ hipError_t launch_refine(hipStream_t stream, int32_t levels_per_lane, const doub
 // consecutive levels each.
 // bins == nullptr: tasks[0, n_tasks) in order; else `bins` (device, 9
 // offsets) splits the list per XCD and `max_bin` is the largest bin's size.
-hipError_t launch_refine_segmented(hipStream_t stream, int32_t lanes, int32_t levels_per_block, const double* uv,
+// simds: the device's SIMDs.
+hipError_t launch_refine_segmented(hipStream_t stream, int32_t simds, int32_t lanes, int32_t levels_per_block,
+                                   const double* uv,
                                    const double* segtab, const PotentialRecord* pots,
                                    const BandWindow* windows, const WaveTask* tasks, int32_t n_tasks,
                                    const int32_t* bins, int32_t max_bin, const Bracket* brackets,
@@ -2693,43 +2698,48 @@ hipError_t launch_refine_segmented(hipStream_t stream, int32_t lanes, int32_t le
     if (levels_per_block != 1 && !((levels_per_block == 2 || levels_per_block == 4) && lanes == 64))
         return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(bins == nullptr ? n_tasks : 8 * max_bin));
-#define EPSEON_SEGMENTED(T, TAB, K)                                                                   \
-    hipLaunchKernelGGL((numerov_refine_segmented_kernel<T, TAB, K>), grid, dim3(T), 0, stream, uv,   \
+    const bool few = static_cast<int64_t>(n_tasks) * (lanes / 64) <= 2 * static_cast<int64_t>(simds);
+#define EPSEON_SEGMENTED(T, TAB, K, W)                                                                 \
+    hipLaunchKernelGGL((numerov_refine_segmented_kernel<T, TAB, K, W>), grid, dim3(T), 0, stream, uv,  \
                        segtab, pots, windows, tasks, n_tasks, bins, brackets, points, rel_tol, max_iter, \
                        levels, status, iterations, steps)
+#define EPSEON_WIDE(T)                        \
+    if (segtab != nullptr && few)             \
+        EPSEON_SEGMENTED(T, true, 1, 2);      \
+    else if (segtab != nullptr)               \
+        EPSEON_SEGMENTED(T, true, 1, 3);      \
+    else if (few)                             \
+        EPSEON_SEGMENTED(T, false, 1, 2);     \
+    else                                      \
+        EPSEON_SEGMENTED(T, false, 1, 3)
     switch (lanes) {
     case 256:
-        if (segtab != nullptr)
-            EPSEON_SEGMENTED(256, true, 1);
-        else
-            EPSEON_SEGMENTED(256, false, 1);
+        EPSEON_WIDE(256);
         break;
     case 128:
-        if (segtab != nullptr)
-            EPSEON_SEGMENTED(128, true, 1);
-        else
-            EPSEON_SEGMENTED(128, false, 1);
+        EPSEON_WIDE(128);
         break;
     case 64:
         if (levels_per_block == 4) {
             if (segtab != nullptr)
-                EPSEON_SEGMENTED(64, true, 4);
+                EPSEON_SEGMENTED(64, true, 4, 2);
             else
-                EPSEON_SEGMENTED(64, false, 4);
+                EPSEON_SEGMENTED(64, false, 4, 2);
         } else if (levels_per_block == 2) {
             if (segtab != nullptr)
-                EPSEON_SEGMENTED(64, true, 2);
+                EPSEON_SEGMENTED(64, true, 2, 3);
             else
-                EPSEON_SEGMENTED(64, false, 2);
+                EPSEON_SEGMENTED(64, false, 2, 3);
         } else if (segtab != nullptr) {
-            EPSEON_SEGMENTED(64, true, 1);
+            EPSEON_SEGMENTED(64, true, 1, 3);
         } else {
-            EPSEON_SEGMENTED(64, false, 1);
+            EPSEON_SEGMENTED(64, false, 1, 3);
         }
         break;
     default:
         return hipErrorInvalidValue;
     }
+#undef EPSEON_WIDE
 #undef EPSEON_SEGMENTED
     return hipGetLastError();
 }
