@@ -335,6 +335,10 @@ def _offsets(points: Sequence[int]) -> np.ndarray:
     return offsets
 
 
+# Larger table buffers are given back when their load ends.
+_KEPT_TABLE_BYTES = 256 << 20
+
+
 class Context:
     """One device context (stream + arena) of libepseon_hip."""
 
@@ -373,12 +377,14 @@ class Context:
         values = [_as_f64(p.values) for p in potentials]
         points = [len(v) for v in values]
         offsets = _offsets(points)
-        # One table buffer per context, kept while it is large enough: a new
-        # one of this size costs more in page faults than the copy.
+        # The context keeps its table buffer for the next load: a new one costs
+        # more in page faults than the copy.  During the call it is this load's
+        # alone.
         total = sum(points)
-        if len(self._tables) < total:
-            self._tables = np.empty(total, dtype=np.float64)
-        v = self._tables[: max(total, 1)]
+        tables, self._tables = self._tables, np.empty(1, dtype=np.float64)
+        if len(tables) < total:
+            tables = np.empty(total, dtype=np.float64)
+        v = tables[: max(total, 1)]
         if total > 0:
             np.concatenate(values, out=v)
         desc = _descriptors(potentials, points)
@@ -392,6 +398,8 @@ class Context:
             )
         )
         self._loaded(desc, points, offsets)
+        if tables.nbytes <= _KEPT_TABLE_BYTES:
+            self._tables = tables
 
     def load_device(self, potentials: Sequence[Potential], v_ptr: int, offsets: Sequence[int]) -> None:
         """Upload a batch whose V tables are already in device memory at
