@@ -171,20 +171,29 @@ def _morse_terms(d: torch.Tensor, de: torch.Tensor, a: torch.Tensor) -> tuple[to
 
 def _plain_tensor(t: torch.Tensor) -> bool:
     """Whether t's memory holds its values: an ordinary dense tensor, not a
-    batched, negated or zero one."""
+    batched, negated or zero one.  False where torch lacks one of the private
+    queries that tell."""
     if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
         return False
-    wrapped = torch._C._functorch
-    return (t.layout is torch.strided and not t.is_neg() and not t._is_zerotensor()
-            and not wrapped.is_functorch_wrapped_tensor(t) and not wrapped.is_legacy_batchedtensor(t))
+    try:
+        wrapped = torch._C._functorch
+        return (t.layout is torch.strided and not t.is_neg() and not t._is_zerotensor()
+                and not wrapped.is_functorch_wrapped_tensor(t) and not wrapped.is_legacy_batchedtensor(t))
+    except AttributeError:
+        return False
 
 
 def _eager() -> bool:
     """No tracer, transform, mode or forward-mode level is active: they see
-    tensor operations, not a kernel."""
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch.autograd.forward_ad._current_level >= 0)
+    tensor operations, not a kernel.  False where torch lacks one of the
+    private queries."""
+    try:
+        return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
+                    or torch._C._are_functorch_transforms_active()
+                    or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                    or torch.autograd.forward_ad._current_level >= 0)
+    except AttributeError:
+        return False
 
 
 def _morse_kernel_takes(r: torch.Tensor, de: torch.Tensor, a: torch.Tensor, re: torch.Tensor) -> bool:
