@@ -223,11 +223,9 @@ def _morse_forward(r: torch.Tensor, de: torch.Tensor, a: torch.Tensor, re: torch
                    v: torch.Tensor, d: torch.Tensor | None) -> None:
     de, a, re = de.contiguous(), a.contiguous(), re.contiguous()
     with torch.cuda.device(r.device):
-        rc = capi.load_library().epseon_morse_table(
+        capi._check(capi.load_library().epseon_morse_table(
             r.data_ptr(), de.data_ptr(), a.data_ptr(), re.data_ptr(), r.shape[0], r.shape[1], v.data_ptr(),
-            None if d is None else d.data_ptr(), torch.cuda.current_stream().cuda_stream)
-    if rc != 0:
-        raise RuntimeError(f"epseon_morse_table failed ({rc})")
+            None if d is None else d.data_ptr(), torch.cuda.current_stream().cuda_stream))
 
 
 class _MorseTable(torch.autograd.Function):
@@ -270,11 +268,9 @@ class _MorseTable(torch.autograd.Function):
         grad = torch.empty((3, rows), dtype=torch.float64, device=d.device)
         part = torch.empty(3 * rows * chunks if chunks > 1 else 0, dtype=torch.float64, device=d.device)
         with torch.cuda.device(d.device):
-            rc = lib.epseon_morse_vjp(g.data_ptr(), d.data_ptr(), de.data_ptr(), a.data_ptr(), rows, points,
-                                      part.data_ptr() or None, grad.data_ptr(),
-                                      torch.cuda.current_stream().cuda_stream)
-        if rc != 0:
-            raise RuntimeError(f"epseon_morse_vjp failed ({rc})")
+            capi._check(lib.epseon_morse_vjp(g.data_ptr(), d.data_ptr(), de.data_ptr(), a.data_ptr(), rows, points,
+                                             part.data_ptr() or None, grad.data_ptr(),
+                                             torch.cuda.current_stream().cuda_stream))
         return grad.unbind(0)
 
 

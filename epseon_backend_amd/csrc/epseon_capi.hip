@@ -61,9 +61,7 @@ hipError_t launch_level_vjp(hipStream_t, int32_t, const double*, const double*,
                             const int32_t*, const LevelNorm*, const PsiCheckpoint*, const double*,
                             double*);
 
-namespace {
-
-thread_local std::string g_last_error;
+static thread_local std::string g_last_error;
 
 int fail(int code, const std::string& msg)
 {
@@ -75,6 +73,8 @@ int hip_fail(hipError_t e, const char* what)
 {
     return fail(EPSEON_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
+
+namespace {
 
 #define EPSEON_HIP_TRY(expr)                                 \
     do {                                                     \

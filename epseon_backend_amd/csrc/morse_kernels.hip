@@ -18,6 +18,7 @@
 #include <cstdint>
 
 #include "epseon_hip.h"
+#include "records.hpp"
 
 namespace epseon::hip {
 
@@ -142,9 +143,10 @@ int64_t morse_chunks(const int64_t rows, const int64_t points)
     return chunks <= kMorseMaxBlocks / rows ? chunks : 0;
 }
 
-int launched()
+int launched(const char* what)
 {
-    return hipGetLastError() == hipSuccess ? EPSEON_OK : EPSEON_ERR_DEVICE;
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? EPSEON_OK : hip_fail(e, what);
 }
 
 }  // namespace
@@ -164,10 +166,10 @@ int epseon_morse_table(const double* r, const double* de, const double* a, const
     using namespace epseon::hip;
     const int64_t chunks = morse_chunks(rows, points);
     if (chunks == 0 || r == nullptr || de == nullptr || a == nullptr || re == nullptr || v == nullptr)
-        return EPSEON_ERR_INVALID;
+        return fail(EPSEON_ERR_INVALID, "epseon_morse_table: null pointer or sizes that no launch takes");
     hipLaunchKernelGGL(morse_table_kernel, dim3(static_cast<unsigned>(rows * chunks)), dim3(kMorseLanes), 0,
                        static_cast<hipStream_t>(stream), r, de, a, re, points, static_cast<uint32_t>(chunks), v, d);
-    return launched();
+    return launched("epseon_morse_table");
 }
 
 int epseon_morse_vjp(const double* g, const double* d, const double* de, const double* a, int64_t rows,
@@ -177,14 +179,14 @@ int epseon_morse_vjp(const double* g, const double* d, const double* de, const d
     const int64_t chunks = morse_chunks(rows, points);
     if (chunks == 0 || g == nullptr || d == nullptr || de == nullptr || a == nullptr || grad == nullptr ||
         (chunks > 1 && part == nullptr))
-        return EPSEON_ERR_INVALID;
+        return fail(EPSEON_ERR_INVALID, "epseon_morse_vjp: null pointer or sizes that no launch takes");
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const uint32_t c = static_cast<uint32_t>(chunks);
     hipLaunchKernelGGL(morse_vjp_kernel, dim3(static_cast<unsigned>(rows * chunks)), dim3(kMorseLanes), 0, s, g, d, de,
                        a, points, c, chunks > 1 ? part : grad);
     if (chunks > 1)
         hipLaunchKernelGGL(morse_sum_kernel, dim3(static_cast<unsigned>(rows)), dim3(kMorseLanes), 0, s, part, c, grad);
-    return launched();
+    return launched("epseon_morse_vjp");
 }
 
 }  // extern "C"

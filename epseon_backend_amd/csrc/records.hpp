@@ -7,9 +7,17 @@
 // offsets into them.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include <cstdint>
+#include <string>
 
 namespace epseon::hip {
+
+// A failing entry point's status code, and its message for
+// epseon_last_error; hip_fail names the call and the HIP error.
+int fail(int code, const std::string& msg);
+int hip_fail(hipError_t e, const char* what);
 
 // Rescale thresholds of the recurrences: the refinement shots multiply the
 // last values by 2^-480 when |w| reaches 2^480; the scan shots (whose values
