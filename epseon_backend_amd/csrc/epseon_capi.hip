@@ -2183,6 +2183,9 @@ int fetch_levels(epseon_ctx* ctx)
         ctx->h_status = reinterpret_cast<const int32_t*>(at(ctx->d_status));
         ctx->h_iters = reinterpret_cast<const int32_t*>(at(ctx->d_iters));
         std::memcpy(ctx->h_summary, at(ctx->d_summary), sizeof ctx->h_summary);
+    } else {
+        // Nothing was refined, and no kernel wrote a summary.
+        std::fill(std::begin(ctx->h_summary), std::end(ctx->h_summary), int64_t(0));
     }
     ctx->host_levels_valid = true;
     return EPSEON_OK;
