@@ -42,6 +42,8 @@ REFINE_SEGMENTED = 2
 
 MEM_HOST = 0
 MEM_DEVICE = 1
+PATH_WIDE_TABLES = 1
+PATH_PACKED_PSI = 2
 
 
 class EpseonError(RuntimeError):
@@ -120,7 +122,7 @@ class Stats(ctypes.Structure):
         ("scan_windows", ctypes.c_int32),
         ("solve_graph", ctypes.c_int32),
         ("refine_levels_per_block", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("paths", ctypes.c_int32),
     ]
 
 

@@ -1615,6 +1615,13 @@ hipError_t wait_tables(epseon_ctx* ctx, hipStream_t stream, int32_t mode, int32_
     return build_tables(ctx, stream, ctx->scan_windows);
 }
 
+// Whether blocks of `lanes` lanes refine through the wide segment tables in
+// the windows of the last scan.
+bool wide_tables(const epseon_ctx* ctx, int32_t lanes)
+{
+    return lanes > 64 && lanes == ctx->wide_lanes && ctx->scan_windows == ctx->wide_band;
+}
+
 // Refinement of the levels of potentials [k0, k1) in task order, in the
 // windows of the last scan.  Lane mode with one level per lane runs the
 // 64-level tasks on `stream`; with two, the paired tasks (potentials with
@@ -1662,7 +1669,7 @@ hipError_t run_refine(epseon_ctx* ctx, hipStream_t stream, hipStream_t stream_b,
     const double* tab = nullptr;
     if (lanes == 64 && ctx->segtab_ok)
         tab = ctx->scan_windows ? ctx->d_segtab_band : ctx->d_segtab_full;
-    else if (lanes == ctx->wide_lanes && ctx->scan_windows == ctx->wide_band)
+    else if (wide_tables(ctx, lanes))
         tab = ctx->d_segtab_wide;
     const bool whole = ctx->xcd_scan && k0 == 0 && k1 == ctx->cum_level_tasks.size() - 1;
     const int32_t lpb = segmented_levels(ctx, lanes), simds = 4 * ctx->compute_units;
@@ -2562,6 +2569,10 @@ int epseon_get_stats(epseon_ctx* ctx, epseon_stats* stats)
         stats->refine_mode = ctx->last_refine_mode;
         stats->refine_lanes = ctx->last_refine_lanes;
         stats->refine_levels_per_block = ctx->last_refine_mode == EPSEON_REFINE_SEGMENTED ? ctx->last_refine_levels : 1;
+        if (ctx->last_refine_mode == EPSEON_REFINE_SEGMENTED && wide_tables(ctx, ctx->last_refine_lanes))
+            stats->paths |= EPSEON_PATH_WIDE_TABLES;
+        if ((ctx->normalize_timed || ctx->vjp_timed) && psi_packed(ctx))
+            stats->paths |= EPSEON_PATH_PACKED_PSI;
         // Eigenfunction passes shoot every converged level once over its
         // trimmed grid (n - 2 steps split between the two inward shots).
         const double shot_pu = static_cast<double>(ctx->h_summary[2]);

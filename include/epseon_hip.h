@@ -108,6 +108,10 @@ typedef struct epseon_potential_info {
     int32_t reserved;
 } epseon_potential_info;
 
+/* ---- kernel variants that a batch's size chose (epseon_stats.paths) ----- */
+#define EPSEON_PATH_WIDE_TABLES 1 /* the refinement's 128- or 256-lane blocks read segment tables */
+#define EPSEON_PATH_PACKED_PSI 2  /* the normalisation packed (segment, level) pairs into wavefronts */
+
 /* Counters and device times of the last calls on a context. */
 typedef struct epseon_stats {
     double scan_ms;               /* device time of the last epseon_scan (HIP events) */
@@ -127,8 +131,8 @@ typedef struct epseon_stats {
     double solve_split;           /* scan-work fraction of the first pipeline group (0: sequential) */
     int32_t scan_windows;         /* 1 when the last scan (and its refinement) used band windows */
     int32_t solve_graph;          /* 1 when the last epseon_solve replayed a captured HIP graph */
-    int32_t refine_levels_per_block; /* levels sharing a block in the last segmented refine (1 or 2) */
-    int32_t reserved;
+    int32_t refine_levels_per_block; /* levels sharing a block in the last segmented refine (1, 2 or 4) */
+    int32_t paths;                /* EPSEON_PATH_* that the last calls took */
 } epseon_stats;
 
 typedef struct epseon_ctx epseon_ctx;
