@@ -187,8 +187,10 @@ constexpr int64_t kDeviceStatsMinPoints = 100000;
 
 // Scans of at most this many wavefronts per SIMD, of whole grids or of at least
 // this many steps on average, spread over the SIMDs as scan_shape says.
-constexpr int64_t kSpreadMaxScanWavesPerSimd = 48;
-constexpr double kSpreadMinSteps = 4096.0;
+// Where the longest shot is over kSpreadEven times the average one, the limit
+// is the lower one.
+constexpr int64_t kSpreadMaxScanWavesPerSimd = 48, kSpreadMaxRaggedWavesPerSimd = 32;
+constexpr double kSpreadMinSteps = 4096.0, kSpreadEven = 3.0;
 
 // Tasks at the end of a windowed scan's bins that are ordered longest first
 // across potentials: four times what an XCD holds at two wavefronts per SIMD.
@@ -455,6 +457,7 @@ struct epseon_ctx {
     bool scan_timed = false, refine_timed = false, normalize_timed = false, vjp_timed = false;
     double scan_point_updates = 0.0;       // of the last scan
     double scan_pu_full = 0.0, scan_pu_band = 0.0;
+    int32_t scan_longest_full = 0, scan_longest_band = 0;  // steps of the longest shot
     std::vector<BandWindow> h_win_full, h_win_band;
 
     explicit epseon_ctx(size_t block_bytes) : arena(block_bytes) {}
@@ -906,7 +909,7 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     }
 
     int64_t pts = 0, en = 0, lv = 0, psi_total = 0, seg_total = 0, ckpt_total = 0, ckpt_long = 0;
-    int32_t max_seg_rows = 0, longest = 0;
+    int32_t max_seg_rows = 0, longest = 0, scan_longest = 0;
     double scan_pu = 0.0;
     for (int32_t p = 0; p < count; ++p) {
         const epseon_potential_desc& d = desc[p];
@@ -985,13 +988,16 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
         pts += ((d.n_points + 7) & ~int64_t(7)) + 64;
         en += d.n_energies;
         lv += d.level_count;
-        if (r.flags == EPSEON_POT_OK)
+        if (r.flags == EPSEON_POT_OK) {
             scan_pu += static_cast<double>(r.n_points - 2) * static_cast<double>(d.n_energies);
+            scan_longest = std::max(scan_longest, r.n_points - 2);
+        }
     }
     ctx->total_points = pts;
     ctx->total_energies = en;
     ctx->total_levels = lv;
     ctx->scan_pu_full = scan_pu;
+    ctx->scan_longest_full = scan_longest;
     ctx->user_span = user_span;
     ctx->psi_total = psi_total;
 
@@ -1387,6 +1393,8 @@ int load_batch(epseon_ctx* ctx, int32_t count, const epseon_potential_desc* desc
     }
     EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max(ctx->n_scan_tasks, 1)), &ctx->d_xcd_scan_tasks_band));
     ctx->scan_pu_band = scan_pu_band;
+    ctx->scan_longest_band =
+        band_task_work.empty() ? 0 : *std::max_element(band_task_work.begin(), band_task_work.end());
     ctx->segtab_ok = max_rows <= INT32_MAX / 512;
     EPSEON_HIP_TRY(arena_array(a, static_cast<size_t>(std::max<int64_t>(band_total, 1)) * 64, &ctx->d_segtab_band));
     ctx->n_jobs_full = static_cast<int32_t>(jobs_full.size());
@@ -1562,10 +1570,14 @@ const BandWindow* scan_window_set(const epseon_ctx* ctx)
 // tables beside them): enough to fill the issue slots, and the rest goes to
 // the SIMDs that come free.  Measured, tuning's value against this one:
 // 8.8 wavefronts per SIMD (256 ragged potentials) 0.94 and 0.76 ms, 8.0 (512 x
-// 50,000 points) 2.78 and 2.32, 18 (512 ragged) 1.60 and 1.31, 37 (1,024) 3.05
-// and 2.94, 72 (2,048) 5.57 and 5.68; whole grids, 5.1 per SIMD 1.05 and 0.88,
+// 50,000 points) 2.78 and 2.32, 18 (512 ragged) 1.64 and 1.40, 23 (640) 1.80
+// and 1.72, 28 (768) 2.21 and 2.18; whole grids, 5.1 per SIMD 1.05 and 0.88,
 // one 1.73 and 1.69.  Windowed shots of 1,500 steps lose (0.30 and 0.33 ms): a
-// workgroup holds its place until its longest wavefront ends.
+// workgroup holds its place until its longest wavefront ends.  So do the many
+// wavefronts of ragged potentials (longest shot six times the average), 32
+// (896) 2.54 and 2.58, 37 (1,024) 2.83 and 2.90, 46 (1,280) 3.61 and 3.80, but
+// not those of equal grids (twice the average), 38 (256 x 50,000 points) 7.60
+// and 7.41, 45 (256 x 20,000) 3.66 and 3.54.
 struct ScanShape {
     int32_t waves, lds;
 };
@@ -1574,7 +1586,9 @@ ScanShape scan_shape(const epseon_ctx* ctx)
 {
     const int64_t simds = 4 * static_cast<int64_t>(ctx->compute_units);
     const double steps = ctx->scan_point_updates / (64.0 * std::max(ctx->n_scan_tasks, 1));
-    const bool spread = ctx->waves_per_block == 1 && ctx->n_scan_tasks <= kSpreadMaxScanWavesPerSimd * simds &&
+    const double longest = ctx->scan_windows ? ctx->scan_longest_band : ctx->scan_longest_full;
+    const int64_t most = longest <= kSpreadEven * steps ? kSpreadMaxScanWavesPerSimd : kSpreadMaxRaggedWavesPerSimd;
+    const bool spread = ctx->waves_per_block == 1 && ctx->n_scan_tasks <= most * simds &&
                         (!ctx->scan_windows || steps >= kSpreadMinSteps);
     return spread ? ScanShape{4, 60 << 10} : ScanShape{ctx->waves_per_block, 0};
 }

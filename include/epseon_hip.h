@@ -258,8 +258,9 @@ typedef struct epseon_tuning {
     int32_t refine_mode;          /* EPSEON_REFINE_* */
     int32_t levels_per_lane;      /* lane mode: 1, or 2 for potentials with more than 64 levels */
     int32_t scan_waves_per_block; /* wavefronts per scan workgroup, 1..4; with 1 (default) scans of up
-                                     to 48 wavefronts per SIMD (whole grids, or windows of 4096 steps
-                                     and more on average) run in workgroups of 4, two per compute unit */
+                                     to 48 wavefronts per SIMD (32 of ragged potentials; whole grids, or
+                                     windows of 4096 steps and more on average) run in workgroups of 4,
+                                     two per compute unit */
     int32_t segmented_lanes;      /* segmented mode: 0 (from the batch size), 64, 128 or 256 */
     int32_t xcd_scan;             /* 1: whole-batch scans and segmented refinements bin potentials per
                                      XCD (default), 0: in order */
