@@ -163,12 +163,6 @@ def uniform_grid(r_min: torch.Tensor, r_max: torch.Tensor, n: int) -> torch.Tens
     return r_min[:, None] + i[None, :] * h[:, None]
 
 
-def _morse_terms(d: torch.Tensor, de: torch.Tensor, a: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-    """V = D_e x^2 and x = 1 - exp(-a d) for d = r - r_e."""
-    x = 1.0 - torch.exp(-a[:, None] * d)
-    return de[:, None] * x * x, x
-
-
 def _plain_tensor(t: torch.Tensor) -> bool:
     """Whether t's memory holds its values: an ordinary dense tensor, not a
     batched, negated or zero one.  False where torch lacks one of the private
@@ -282,4 +276,5 @@ def morse_table(r: torch.Tensor, de: torch.Tensor, a: torch.Tensor, re: torch.Te
         v = torch.empty_like(r)
         _morse_forward(r, de, a, re, v, None)
         return v
-    return _morse_terms(r - re[:, None], de, a)[0]
+    x = 1.0 - torch.exp(-a[:, None] * (r - re[:, None]))
+    return de[:, None] * x * x

@@ -1514,12 +1514,12 @@ int32_t segmented_lanes(const epseon_ctx* ctx)
 // Whether the normalisation's segment pass packs a potential's (segment,
 // level) pairs into full wavefronts: when that takes at least a sixteenth of
 // the wavefronts away and each SIMD has kPsiPackTasks / 1024 of them, so that
-// their number is what the pass costs.  256 x 50,000 points with 41 levels 581
-// -> 416 us; 96 x 50,000 points (normalisation, both passes): 17 levels 244 ->
-// 120 us, 48 levels 261 -> 224, 60 levels 270 -> 259, 68 levels 1,195 -> 285;
-// 41 levels on 32 x 50,000 points 112 -> 95, but on 64 x 10,000 points (5,000
-// tasks) 56 -> 58 and on 16 x 50,000 (3,100) 65 -> 67: lanes that load their
-// own values wait for vector loads.
+// their number is what the pass costs.  Normalisation, both passes: 256 x
+// 50,000 points with 41 levels 600 -> 470 us; 96 x 50,000 points: 17 levels 233
+// -> 110, 48 levels 247 -> 216, 60 levels 253 -> 253, 68 levels 486 -> 280; 41
+// levels on 128 x 10,000 points (8,100 tasks) 78 -> 69, on 32 x 50,000 (5,000)
+// 101 -> 93, but on 64 x 10,000 (4,000) 48 -> 50 and on 16 x 50,000 (2,500) 68
+// -> 71: lanes that load their own values wait for vector loads.
 constexpr int64_t kPsiPackTasks = 6144;
 bool psi_packed(const epseon_ctx* ctx)
 {

@@ -30,11 +30,12 @@
 // Kernels in this file, in launch order: potential statistics and table
 // shifts (load), band windows (each shot stops 15 guaranteed e-folds past its
 // band top's outermost turning points), segment tables (load), the scan, the
-// bracket pass (one thread per level), and the refinement: lane mode (one
-// level per lane over the whole grid) or segmented mode (one block per level,
-// each lane a segment's transfer matrix, tree product in LDS, 64-lane blocks
-// reading the per-window segment table).  Scan and segmented tasks are binned
-// per XCD so that a potential's wavefronts share one L2.
+// bracket pass (a 16-lane row per level), and the refinement: lane mode (one
+// level per lane over the whole grid) or segmented mode (a block of 64 to 256
+// lanes per level or group of levels, each lane a segment's transfer matrix,
+// tree product in registers or LDS, reading the per-window segment tables; in
+// wide blocks of short grids the natural table).  Scan and segmented tasks are
+// binned per XCD so that a potential's wavefronts share one L2.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -761,9 +762,12 @@ __device__ constexpr double kGrowthRatio[9] = {65450, 65366, 65199, 64871, 64242
 // sqrt(T 2^r) 2^h (k + 64 = 2 h + r) is taken as isqrt(T 2^(r+32)) 2^(h-16),
 // floored, times the growth ratio at 2^k (the ratio falls with y; entry -5
 // serves below) over 65536.  Whole numbers held in doubles: T and k come from
-// the bits of x, every product has at most 41 significant bits and every sum
-// of terms stays below 2^53, so all of it is exact.  0 below 2^-65; x >= 8
-// counts as just below 8.  `ratio`: kGrowthRatio in LDS.  About 30
+// the bits of x, and every product has at most 41 significant bits, so each
+// term is exact.  So are sums up to 2^53: those of a wavefront's 512 terms
+// (below 2^51), and whatever a walk adds up before it reaches the depth (below
+// 2^44).  A step of sixteen wavefronts can add up to 2^54 and round, but only
+// far past the depth, where it still compares as past it.  0 below 2^-65; x >=
+// 8 counts as just below 8.  `ratio`: kGrowthRatio in LDS.  About 30
 // instructions where 64-bit integers took four times as many.
 __device__ __forceinline__ double growth_term(const double x, const double* ratio)
 {

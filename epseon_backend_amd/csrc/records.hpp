@@ -87,8 +87,8 @@ constexpr int32_t load_chunks(const int64_t n_points, const int32_t least)
     return static_cast<int32_t>((n_points + c - 1) / c);
 }
 
-// Minimum of one chunk of a V table: value, first index (n_points if the
-// chunk has no finite value) and first non-finite index (n_points if none).
+// Minimum of one chunk of a V table: value, first index (INT64_MAX if the
+// chunk has no finite value) and first non-finite index (INT64_MAX if none).
 struct ChunkMin {
     double vmin;
     int64_t imin, bad;
